@@ -190,24 +190,39 @@ __device__ __forceinline__ void zero_tally_lds(int* s_red) {
   for (int i = threadIdx.x; i <= kTallyWidth; i += blockDim.x) s_red[i] = 0;
 }
 
-// Folds the slots into the step's row and into the running totals (and
-// counts the step), clearing the slots; clears `flux_next` (nflux values),
-// the flux statistics buffer of the next BE step, when it is not null.
-__global__ void k_tally_close(unsigned long long* slots, unsigned long long* row, unsigned long long* totals,
-                              int steps, double* flux_next, int nflux) {
-  for (int c = threadIdx.x; c < kTallyWidth; c += blockDim.x) {
+// Where a step's counters go: folds the slots into the step's row and into
+// the running totals (and counts the step), clearing the slots; clears
+// `flux_next` (nflux values), the flux statistics buffer of the next BE step,
+// when it is not null.
+struct TallyClose {
+  unsigned long long *slots, *row, *totals;
+  int steps;
+  double* flux_next;
+  int nflux;
+};
+// thread i of nt
+__device__ __forceinline__ void close_tally(const TallyClose& tc, int i, int nt) {
+  for (int c = i; c < kTallyWidth; c += nt) {
     unsigned long long s = 0;
-    for (int k = 0; k < kTallySlots; ++k) {
-      s += slots[k * kTallyWidth + c];
-      slots[k * kTallyWidth + c] = 0ull;
+#pragma unroll 1  // a few registers, whatever kernel this is part of
+    for (int k0 = 0; k0 < kTallySlots; k0 += 8) {
+      unsigned long long v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = tc.slots[(k0 + k) * kTallyWidth + c];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        s += v[k];
+        tc.slots[(k0 + k) * kTallyWidth + c] = 0ull;
+      }
     }
-    s += (c == kTSteps ? (unsigned long long)steps : 0ull);
-    row[c] = s;
-    totals[c] += s;
+    s += (c == kTSteps ? (unsigned long long)tc.steps : 0ull);
+    tc.row[c] = s;
+    tc.totals[c] += s;
   }
-  if (flux_next)
-    for (int i = threadIdx.x; i < nflux; i += blockDim.x) flux_next[i] = 0.0;
+  if (tc.flux_next)
+    for (int k = i; k < tc.nflux; k += nt) tc.flux_next[k] = 0.0;
 }
+__global__ void k_tally_close(TallyClose tc) { close_tally(tc, threadIdx.x, blockDim.x); }
 
 // ------------------------------------------------------------ load/store
 
@@ -1345,11 +1360,20 @@ __global__ void k_xy_reduce(const double* part, int rows, int width, double* out
   out[i] = v;
 }
 
-// Exclusive scan of the u-cell histogram: per-block sums, one-block scan of
-// the block sums, then a block-local scan with the block's prefix.
+// Exclusive scan of the u-cell histogram: k_scan_reduce sums its tiles, then
+// k_scan_down<true> scans every tile locally and adds up the sums of the tiles
+// before it itself, which is cheaper than a launch (4.6 us) for a one-workgroup
+// scan of the sums up to kScanDirect tiles (1.3e8 cells; there the last
+// workgroups read 64 KB each); beyond, k_scan_bsum scans the sums and
+// k_scan_down<false> takes its tile's prefix from them.  With the counters
+// closed on the way, two launches a step fewer: 64^3 with 100k droplets (FP64)
+// 2100 -> 1982 us for 20 steps, 1000 droplets 684 -> 625 us for 10.  (Tile sums kept by the
+// step kernel, one atomic per wave and tile, made it 2 % slower at 20M droplets
+// and 9 % at 333k: every wave in flight adds to the same few words.)
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
+constexpr int64_t kScanDirect = 16384;
 
 __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave, int& total) {
   const int lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -1377,8 +1401,15 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave, int& tot
   return before + x - v;
 }
 
-__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const int32_t* in, int64_t n, int32_t* bsum) {
+// The workgroup after the last tile, when launched, closes the counters of the
+// step before (a launch of its own otherwise).
+__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const int32_t* in, int64_t n, int32_t* bsum,
+                                                              TallyClose tc) {
   __shared__ int s_wave[16];
+  if ((int64_t)blockIdx.x * kScanTile >= n) {
+    close_tally(tc, threadIdx.x, blockDim.x);
+    return;
+  }
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   int v = 0;
 #pragma unroll
@@ -1404,9 +1435,18 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_bsum(int32_t* bsum, int64
   }
 }
 
+template <bool DIRECT>
 __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int32_t* in, int64_t n, const int32_t* bsum,
                                                             int32_t* out) {
   __shared__ int s_wave[16];
+  int before;  // the counts before this tile
+  if (DIRECT) {
+    int v = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanThreads) v += bsum[b];
+    (void)block_exclusive_scan(v, s_wave, before);
+  } else {
+    before = bsum[blockIdx.x];
+  }
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   // thread-contiguous items for a cheap serial prefix
   const int64_t i0 = base + (int64_t)threadIdx.x * kScanItems;
@@ -1426,7 +1466,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int32_t* in, i
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) sum += v[k];
   int total;
-  int run = block_exclusive_scan(sum, s_wave, total) + bsum[blockIdx.x];
+  int run = block_exclusive_scan(sum, s_wave, total) + before;
   int o[kScanItems];
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
@@ -1442,7 +1482,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int32_t* in, i
       if (i0 + k < n) out[i0 + k] = o[k];
   }
   // grand total at out[n]
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = bsum[blockIdx.x] + total;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + total;
 }
 
 // Counting-sort scatter: slot t goes to offsets[key] + its rank among the

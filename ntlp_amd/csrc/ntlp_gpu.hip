@@ -373,25 +373,29 @@ int upload_consts() {
   return 0;
 }
 
-// exclusive scan counts -> offsets (ncell + 1 entries)
-int scan_counts() {
-  const int64_t nb = (ctx.ncell + kScanTile - 1) / kScanTile;
-  CHK(launch("bin_scan", [&] { k_scan_reduce<<<(unsigned)nb, kScanThreads, 0, ctx.stream>>>(ctx.counts, ctx.ncell, ctx.bsum); }));
-  CHK(launch("bin_scan", [&] { k_scan_bsum<<<1, kScanThreads, 0, ctx.stream>>>(ctx.bsum, nb); }));
-  CHK(launch("bin_scan", [&] {
-    k_scan_down<<<(unsigned)nb, kScanThreads, 0, ctx.stream>>>(ctx.counts, ctx.ncell, ctx.bsum, ctx.offsets);
-  }));
-  return 0;
+// exclusive scan counts -> offsets (ncell + 1 entries) on `stream`; tc: closes
+// the counters of the step before on the way
+void launch_scan(const int32_t* counts, int32_t* bsum, int32_t* offsets, int64_t ncell, const TallyClose* tc,
+                 hipStream_t stream) {
+  const int64_t nb = (ncell + kScanTile - 1) / kScanTile;
+  k_scan_reduce<<<(unsigned)nb + (tc ? 1 : 0), kScanThreads, 0, stream>>>(counts, ncell, bsum, tc ? *tc : TallyClose());
+  if (nb <= kScanDirect) {
+    k_scan_down<true><<<(unsigned)nb, kScanThreads, 0, stream>>>(counts, ncell, bsum, offsets);
+  } else {
+    k_scan_bsum<<<1, kScanThreads, 0, stream>>>(bsum, nb);
+    k_scan_down<false><<<(unsigned)nb, kScanThreads, 0, stream>>>(counts, ncell, bsum, offsets);
+  }
 }
 
 // keys + counts of the current slot order must be in place; leaves perm
-// sorted by u cell (ties by `tie`, or by slot) and counts zeroed.
+// sorted by u cell (ties by `tie`, or by slot) and counts zeroed.  tc: closes
+// the counters of the step before on the way.
 // canonical: order the droplets within each cell by `tie` (or by slot), so
 // that the permutation does not depend on the order of the scatter's
 // atomics.  The fused step does not need that (a droplet's arithmetic does
 // not depend on its slot); the bin queries and the deterministic coupling do.
-int finish_bin(const int32_t* tie, bool canonical = true) {
-  CHK(scan_counts());
+int finish_bin(const int32_t* tie, bool canonical = true, const TallyClose* tc = nullptr) {
+  CHK(launch("bin_scan", [&] { launch_scan(ctx.counts, ctx.bsum, ctx.offsets, ctx.ncell, tc, ctx.stream); }));
   CHK(launch("bin_scatter", [&] {
     k_bin_scatter<<<bin_blocks(ctx.n), kBlock, 0, ctx.stream>>>(ctx.keys[ctx.cur], ctx.n, ctx.offsets, ctx.counts, ctx.perm,
                                                               nullptr);
@@ -691,18 +695,19 @@ int flux_len() { return 3 * (ctx.g.nnz + 1); }
 // flux statistics buffer of BE step j
 double* flux_buf(int64_t j) { return ctx.flux + (j % 2) * flux_len(); }
 
-// closes the current step: slots -> a fresh per-step row and the totals; a
-// BE step also clears the flux buffer of the next BE step
-int close_step(bool be) {
+// where the current step's counters go: a fresh per-step row and the totals;
+// a BE step also clears the flux buffer of the next BE step
+TallyClose next_close(bool be) {
   ctx.step_row++;
-  unsigned long long* row = ctx.tally + (ctx.step_row % kTallyRows) * kTallyWidth;
-  unsigned long long* slots = ctx.tally_slots;
-  unsigned long long* totals = ctx.tally_totals;
-  double* next = be ? flux_buf(ctx.be_steps + 1) : nullptr;
-  const int nf = flux_len();
-  CHK(launch("tally", [&] { k_tally_close<<<1, 128, 0, ctx.stream>>>(slots, row, totals, 1, next, nf); }));
+  TallyClose tc;
+  tc.slots = ctx.tally_slots;
+  tc.row = ctx.tally + (ctx.step_row % kTallyRows) * kTallyWidth;
+  tc.totals = ctx.tally_totals;
+  tc.steps = 1;
+  tc.flux_next = be ? flux_buf(ctx.be_steps + 1) : nullptr;
+  tc.nflux = flux_len();
   if (be) ctx.be_steps++;
-  return 0;
+  return tc;
 }
 
 // nsteps fused steps: each reads the droplets through the cell sort, writes
@@ -729,7 +734,10 @@ int settle(int steps) {
 // one step) and, for BE, its zero flux statistics; the coupling sources are
 // zero.
 int empty_steps(int mode, int nsteps, bool scatter) {
-  for (int k = 0; k < nsteps; ++k) CHK(close_step(mode == NTLP_MODE_BE));
+  for (int k = 0; k < nsteps; ++k) {
+    const TallyClose tc = next_close(mode == NTLP_MODE_BE);
+    CHK(launch("tally", [&] { k_tally_close<<<1, 128, 0, ctx.stream>>>(tc); }));
+  }
   if (scatter) {
     CHK(fill_f64(ctx.src, 6 * ctx.nsrc, 0.0));
     ctx.src_valid = true;
@@ -775,8 +783,8 @@ int run_fused_steps(int mode, int prec, int nsteps, int it0, bool scatter, bool 
     }
     ctx.keys_valid = true;
     done = k + 1;
-    CHK(close_step(mode == NTLP_MODE_BE));
-    CHK(finish_bin(nullptr, false));
+    const TallyClose tc = next_close(mode == NTLP_MODE_BE);
+    CHK(finish_bin(nullptr, false, &tc));
     if (scatter && src_mask()) CHK(tile_sorted());  // no coupling flag: the sources stay zero
   }
   if (lazy) CHK(settle(nsteps));  // the call's residence-time additions

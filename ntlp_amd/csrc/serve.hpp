@@ -276,10 +276,7 @@ void serve_launch_step(const StepArgs& a, unsigned grid) {
 // droplet's arithmetic depends on it), then the step.  Sizes come from the
 // control block.
 void serve_enqueue_step(int64_t size, int cur) {
-  const int64_t nb = (ctx.ncell + kScanTile - 1) / kScanTile;
-  k_scan_reduce<<<(unsigned)nb, kScanThreads, 0, srv.stream>>>(srv.counts, ctx.ncell, srv.bsum);
-  k_scan_bsum<<<1, kScanThreads, 0, srv.stream>>>(srv.bsum, nb);
-  k_scan_down<<<(unsigned)nb, kScanThreads, 0, srv.stream>>>(srv.counts, ctx.ncell, srv.bsum, srv.offsets);
+  launch_scan(srv.counts, srv.bsum, srv.offsets, ctx.ncell, nullptr, srv.stream);
   k_bin_scatter<<<bin_blocks(size), kBlock, 0, srv.stream>>>(srv.keys[cur], size, srv.offsets, srv.counts, srv.perm,
                                                         &srv.ctl_dev->hw);
   const StepArgs a = serve_step_args(cur);
