@@ -459,7 +459,8 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
         rk3_droplet<PREC, ILIN>(a.g, C, a.fl, a.F, s_z, s_zz, d, st, a.it, o, o.kpt, &bx);
     } else {
       // q* is a diagnostic of the record: formed on the step that stores it
-      be_droplet<PREC, ILIN, LAZY>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, kg, SERVE ? nullptr : a.flux,
+      constexpr bool keep = SERVE || PREC != PREC_MIXED || ILIN != 1;  // see lv_solver
+      be_droplet<PREC, ILIN, LAZY, keep>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, kg, SERVE ? nullptr : a.flux,
                                    mult, &bx, !SERVE && a.write_cold);
     }
     if (SERVE && a.serve->last[home >> kServeIdxBits]) {

@@ -274,42 +274,75 @@ __device__ __forceinline__ int gauss_newton(const Ev& ev, const double vec1[2], 
   return flag;
 }
 
+// What a Levenberg-Marquardt iteration needs of a point: J^T J, J^T F and the
+// merit |(F1^2/2, F2^2/2)|.
+__device__ __forceinline__ double lm_merit(const double F[2]) {
+  const double C0 = 0.5 * F[0] * F[0], C1 = 0.5 * F[1] * F[1];
+  return sqrt(C0 * C0 + C1 * C1);
+}
+struct LmPoint {
+  double a00, a01, a11, g0, g1, merit;
+  template <class Ev>
+  __device__ __forceinline__ void evaluate(const Ev& ev, const double v[2]) {
+    double F[2], J[2][2];
+    ev.fj(v[0], v[1], F, J);
+    a00 = J[0][0] * J[0][0] + J[1][0] * J[1][0];
+    a01 = J[0][0] * J[0][1] + J[1][0] * J[1][1];
+    a11 = J[0][1] * J[0][1] + J[1][1] * J[1][1];
+    g0 = J[0][0] * F[0] + J[1][0] * F[1];
+    g1 = J[0][1] * F[0] + J[1][1] * F[1];
+    merit = lm_merit(F);
+  }
+};
+
 // LV_solver (4143-4223): Levenberg-Marquardt, lambda 1e-3 halved on success
-// and doubled otherwise, merit |(F1^2/2, F2^2/2)|.  vec2 keeps what the failed
-// Gauss-Newton left, as the shared actual argument rt_zeroes does.
-template <class Ev>
+// and doubled otherwise.  vec2 keeps what the failed Gauss-Newton left, as the
+// shared actual argument rt_zeroes does.
+//
+// A solve is one serial chain of about 88 iterations, half of them rejected,
+// in a lane or two of a wave that the end of the kernel waits for.  KEEP: each
+// iteration evaluates the equations once, at its candidate, residual and
+// Jacobian together: an accepted candidate's values are the next iteration's,
+// a rejected iteration keeps the old ones.  That halves the chain, for 16
+// registers (a burst of 16 served ensembles, 0.02 % of whose solves fall back:
+// 9.97 -> 9.01 ms); the mixed step of the library, at 123 of the 128 that four waves
+// per SIMD leave, evaluates again instead (KEEP false: 141 registers and three
+// waves cost more than the tail).
+template <bool KEEP, class Ev>
 __device__ __forceinline__ int lv_solver(const Ev& ev, const double vec1[2], double vec2[2], int& iters) {
   int iterations = 0, flag = 0;
   double v1[2] = {vec1[0], vec1[1]};
   double lambda = 0.001;
+  LmPoint at;
+  if (KEEP) at.evaluate(ev, v1);
   while (iterations < 1000) {
     iterations++;
-    double J[2][2], fv1[2];
-    ev.fj(v1[0], v1[1], fv1, J);
-    double gm[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) gm[i][j] = (J[0][i] * J[0][j] + J[1][i] * J[1][j]) + lambda * (i == j ? 1.0 : 0.0);
-    const double gradC0 = J[0][0] * fv1[0] + J[1][0] * fv1[1];
-    const double gradC1 = J[0][1] * fv1[0] + J[1][1] * fv1[1];
-    const double C0 = 0.5 * fv1[0] * fv1[0], C1 = 0.5 * fv1[1] * fv1[1];
-    const double det = gm[0][0] * gm[1][1] - gm[0][1] * gm[1][0];
+    if (!KEEP) at.evaluate(ev, v1);
+    const double gm00 = at.a00 + lambda, gm11 = at.a11 + lambda, gm01 = at.a01;
+    const double det = gm00 * gm11 - gm01 * gm01;
     if (fabs(det) < 1.0e-10) { flag = 1; break; }
     const double s = 1. / det;
-    const double i00 = s * gm[1][1], i10 = s * (-gm[1][0]), i01 = s * (-gm[0][1]), i11 = s * gm[0][0];
-    const double c0 = i00 * gradC0 + i01 * gradC1;
-    const double c1 = i10 * gradC0 + i11 * gradC1;
+    const double i00 = s * gm11, i01 = s * (-gm01), i11 = s * gm00;
+    const double c0 = i00 * at.g0 + i01 * at.g1;
+    const double c1 = i01 * at.g0 + i11 * at.g1;
     vec2[0] = v1[0] - c0;
     vec2[1] = v1[1] - c1;
-    if (sqrt(c0 * c0 + c1 * c1) < 1.0e-8) break;
+    // sqrt(c0^2 + c1^2) < 1e-8: the square root is correctly rounded, and
+    // 1e-16 is the smallest double whose root is not below 1e-8
+    if (c0 * c0 + c1 * c1 < 1.0e-16) break;
     if (vec2[0] < 0.0 || vec2[1] < 0.0 || isnan(vec2[0]) || isnan(vec2[1])) { flag = 1; break; }
-    double fv2[2];
-    ev.f(vec2[0], vec2[1], fv2);
-    const double n0 = 0.5 * fv2[0] * fv2[0], n1 = 0.5 * fv2[1] * fv2[1];
-    if (sqrt(n0 * n0 + n1 * n1) < sqrt(C0 * C0 + C1 * C1)) {
+    LmPoint to;
+    if (KEEP) {
+      to.evaluate(ev, vec2);
+    } else {
+      double F[2];
+      ev.f(vec2[0], vec2[1], F);
+      to.merit = lm_merit(F);
+    }
+    if (to.merit < at.merit) {
       v1[0] = vec2[0];
       v1[1] = vec2[1];
+      if (KEEP) at = to;
       lambda = lambda / 2.0;
     } else {
       lambda = lambda * 2.0;
@@ -441,7 +474,7 @@ __device__ __forceinline__ double rad_solver2_mixed(const DevConsts& C, double T
 // reaches depends on where it starts; a guess formed wholly in FP32
 // (Cardano's discriminant cancels near the Koehler maximum) sent a few
 // hundred droplets per step of the stiff activation case into failed solves.
-template <int PREC>
+template <int PREC, bool KEEP>
 __device__ __forceinline__ void be_microphysics(const DevConsts& C, const DevFlags& fl, Drop& d,
                                                 double Tf, double qinf, double rhoa, double diffnorm,
                                                 double Rep, double esa, Tally& tl) {
@@ -490,7 +523,7 @@ __device__ __forceinline__ void be_microphysics(const DevConsts& C, const DevFla
       if (flag == 1) {
         tl.num100 += 1;
         tl.hist = 0;
-        flag = lv_solver(ev, rt_start, rt_zeroes, it2);
+        flag = lv_solver<KEEP>(ev, rt_start, rt_zeroes, it2);
         tl.lm_iters += it2;
       }
     } else {
@@ -515,7 +548,7 @@ __device__ __forceinline__ void be_microphysics(const DevConsts& C, const DevFla
       if (flag == 1) {
         tl.num100 += 1;
         tl.hist = 0;
-        flag = lv_solver(ev, rt_start, rt_zeroes, it2);
+        flag = lv_solver<KEEP>(ev, rt_start, rt_zeroes, it2);
         tl.lm_iters += it2;
       }
     }
@@ -694,14 +727,14 @@ __device__ __forceinline__ void be_flux(const DevGrid& g, const DevConsts& C, co
 // with_qstar, i.e. when the caller stores it), residence times, flux
 // statistics (flux not null; levels: the packed levels be_advance left), then
 // walls at the new radius.
-template <int PREC, bool LAZY = false>
+template <int PREC, bool LAZY, bool KEEP>
 __device__ __forceinline__ void be_finish(const DevGrid& g, const DevConsts& C, const DevFlags& fl,
                                           const double* s_z, Drop& d, const BeHand& h, double& qstar,
                                           Tally& tl, int levels, double* flux = nullptr, int64_t mult = 1,
                                           bool with_qstar = true) {
   const double dt = C.dt;
   const double esa = (PREC == PREC_FP64) ? mod_magnus(h.Tf) : mod_magnus_fast(h.Tf);
-  be_microphysics<PREC>(C, fl, d, h.Tf, h.qinf, h.rhoa, h.diffnorm, h.Rep, esa, tl);
+  be_microphysics<PREC, KEEP>(C, fl, d, h.Tf, h.qinf, h.rhoa, h.diffnorm, h.Rep, esa, tl);
   qstar = 0.0;
   if (with_qstar)
     qstar = (PREC == PREC_MIXED) ? qstar_f32(C, d, h.Tf, h.rhoa, esa) : qstar_f64(C, d, h.Tf, h.rhoa, esa);
@@ -714,14 +747,14 @@ __device__ __forceinline__ void be_finish(const DevGrid& g, const DevConsts& C, 
 }
 
 // One droplet of particle_update_BE (3043-3238) plus its boundary conditions.
-template <int PREC, int ILIN, bool LAZY = false>
+template <int PREC, int ILIN, bool LAZY = false, bool KEEP = true>
 __device__ __forceinline__ void be_droplet(const DevGrid& g, const DevConsts& C, const DevFlags& fl,
                                            const DevFields& F, const double* s_z, const double* s_zz,
                                            Drop& d, int it, Diag& o, Tally& tl, int kguess = -1,
                                            double* flux = nullptr, int64_t mult = 1,
                                            const FieldBox* bx = nullptr, bool with_qstar = true) {
   const BeHand h = be_advance<PREC, ILIN>(g, C, fl, F, s_z, s_zz, d, it, o, kguess, bx);
-  be_finish<PREC, LAZY>(g, C, fl, s_z, d, h, o.qstar, tl, o.kpt, flux, mult, with_qstar);
+  be_finish<PREC, LAZY, KEEP>(g, C, fl, s_z, d, h, o.qstar, tl, o.kpt, flux, mult, with_qstar);
   o.kpt = packed_kpt(o.kpt);
 }
 
