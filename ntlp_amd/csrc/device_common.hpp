@@ -558,91 +558,145 @@ __device__ FieldBox stage_box(const DevGrid& g, const DevFields& F, int key, boo
   return b;
 }
 
-// uf_interp (particles.f90:554-765): 6th-order Lagrange on 6x6x6 nodes with
-// the reference's one-sided truncation near the walls.  FP64 in all
-// precisions.  The out-of-domain branches with first=last=0 leave the weights
-// zero (the reference evaluates one stray iteration outside its arrays there).
-__device__ __noinline__ Fluid gather6_f64(const DevGrid& g, const DevFields& F, const double* s_z,
-                                          const double* s_zz, double x, double y, double z,
-                                          const Cell& c) {
-  const int nnz = g.nnz;
-  int kuv[6], kwv[6];
-  double wt[4][6];
-  kuv[2] = c.kpt;
-  kuv[3] = kuv[2] + 1; kuv[4] = kuv[3] + 1; kuv[5] = kuv[4] + 1;
-  kuv[1] = kuv[2] - 1; kuv[0] = kuv[1] - 1;
-  kwv[2] = c.kwpt;
-  kwv[3] = kwv[2] + 1; kwv[4] = kwv[3] + 1; kwv[5] = kwv[4] + 1;
-  kwv[1] = kwv[2] - 1; kwv[0] = kwv[1] - 1;
-  for (int a = 0; a < 4; ++a)
-    for (int b = 0; b < 6; ++b) wt[a][b] = 0.0;
-  {
-    const double dxv[2] = {g.dx, g.dy};
-    const double xp[2] = {x, y};
-    const int base[2] = {c.ipt, c.jpt};
-    for (int d = 0; d < 2; ++d)
-      for (int j = 0; j < 6; ++j) {
-        double xj = dxv[d] * (double)(base[d] + j - 3);
-        double pj = 1.0;
-        for (int k = 0; k < 6; ++k) {
-          double xk = dxv[d] * (double)(base[d] + k - 3);
-          if (j != k) pj = pj * (xp[d] - xk) / (xj - xk);
-        }
-        wt[d][j] = pj;
-      }
+// 6-point Lagrange weights of x on the nodes h*(n0), ..., h*(n0 + 5), in the
+// reference's operations (particles.f90:583-597).
+__device__ __forceinline__ void lag_horizontal(double x, double h, int n0, double w[6]) {
+  double xn[6], dx[6];
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    xn[a] = h * (double)(n0 + a);
+    dx[a] = x - xn[a];
   }
-  int first, last;
-  if (kuv[2] == 1) { first = 3; last = 4; kuv[0] = 1; kuv[1] = 1; }
-  else if (kuv[2] == 0) { first = 4; last = 5; kuv[0] = 1; kuv[1] = 1; kuv[2] = 1; }
-  else if (kuv[2] < 0) { first = 0; last = 0; }
-  else if (kuv[2] == 2) { first = 2; last = 5; }
-  else if (kuv[2] == nnz) { first = 2; last = 3; kuv[3] = nnz; kuv[4] = nnz; kuv[5] = nnz; }
-  else if (kuv[2] > nnz) { first = 0; last = 0; }
-  else if (kuv[2] == nnz - 1) { first = 3; last = 4; kuv[4] = nnz; kuv[5] = nnz; }
-  else if (kuv[2] == nnz - 2) { first = 2; last = 5; }
-  else { first = 1; last = 6; }
-  if (first > 0)
-    for (int j = first; j <= last; ++j) {
-      double xj = s_zz[clampi(kuv[j - 1], 0, nnz + 1)];
-      double pj = 1.0;
-      for (int k = first; k <= last; ++k) {
-        double xk = s_zz[clampi(kuv[k - 1], 0, nnz + 1)];
-        if (j != k) pj = pj * (z - xk) / (xj - xk);
-      }
-      wt[2][j - 1] = pj;
-    }
-  if (kwv[2] == 0) { first = 3; last = 4; kwv[0] = 1; kwv[1] = 1; }
-  else if (kwv[2] < 0) { first = 0; last = 0; kwv[0] = 1; kwv[1] = 1; kwv[2] = 1; }
-  else if (kwv[2] == 1) { first = 2; last = 5; kwv[0] = 1; }
-  else if (kwv[2] == nnz - 1) { first = 3; last = 4; kwv[4] = nnz; kwv[5] = nnz; }
-  else if (kwv[2] >= nnz) { first = 0; last = 0; kwv[2] = nnz; kwv[3] = nnz; kwv[4] = nnz; kwv[5] = nnz; }
-  else if (kwv[2] == nnz - 2) { first = 2; last = 5; kwv[5] = nnz; }
-  else { first = 1; last = 6; }
-  if (first > 0)
-    for (int j = first; j <= last; ++j) {
-      double xj = s_z[clampi(kwv[j - 1], 0, nnz + 1)];
-      double pj = 1.0;
-      for (int k = first; k <= last; ++k) {
-        double xk = s_z[clampi(kwv[k - 1], 0, nnz + 1)];
-        if (j != k) pj = pj * (z - xk) / (xj - xk);
-      }
-      wt[3][j - 1] = pj;
-    }
-  Fluid f = {{0.0, 0.0, 0.0}, 0.0, 0.0};
-  for (int k = 0; k < 6; ++k) {
-    const int izuv = clampi(kuv[k], 0, nnz + 1), izw = clampi(kwv[k], 0, nnz + 1);
-    for (int j = 0; j < 6; ++j) {
-      const int iy = clampi(c.jpt + j - 2, -1, g.nny + 3);
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    double p = 1.0;
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+      if (j != k) p = p * dx[k] / (xn[j] - xn[k]);
+    w[j] = p;
+  }
+}
+
+// Lagrange weights of z on the levels lev[k[lo]] .. lev[k[hi]] of the six, zero
+// on the others (hi < lo: all zero), likewise (600-700).
+__device__ __forceinline__ void lag_vertical(const double* lev, const int k[6], int lo, int hi, int kmax, double z,
+                                             double w[6]) {
+  double zn[6], dz[6];
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    zn[a] = lev[clampi(k[a], 0, kmax)];
+    dz[a] = z - zn[a];
+  }
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    double p = 1.0;
+#pragma unroll
+    for (int b = 0; b < 6; ++b)
+      if (j != b) p = (b >= lo && b <= hi) ? p * dz[b] / (zn[j] - zn[b]) : p;
+    w[j] = (j >= lo && j <= hi) ? p : 0.0;
+  }
+}
+
+// uf_interp (particles.f90:554-765): 6th-order Lagrange on 6x6x6 nodes with
+// the reference's one-sided truncation near the walls, in its operations and
+// order of additions, FP64 in all precisions.  The out-of-domain branches with
+// first=last=0 leave the weights zero (the reference evaluates one stray
+// iteration outside its arrays there).
+// The weights stay in registers: every loop over them is unrolled, but for the
+// outermost over three pairs of levels, which shifts its lists down by two each
+// turn.  (Indexed by loop counters they lived in scratch memory, 1.2 KB a
+// droplet.)  The vector cache bounds it: a load of one level by a wave touches
+// about 21 cache lines, and the order of additions has the levels outermost, so
+// both levels of a pair come in one 16-byte load, and the upper one waits in a
+// register until the lower plane is summed.  FP64 step of 700k droplets on
+// 96^3 (280 us of it the tail of its few Levenberg-Marquardt solves): 1480 us
+// with scratch, about 900 with one level a load, 715 now; drawing them, in no
+// order: 11.9, 11.4 and 5.0 ms.
+__device__ __forceinline__ Fluid gather6_f64(const DevGrid& g, const DevFields& F, const double* s_z,
+                                             const double* s_zz, double x, double y, double z,
+                                             const Cell& c) {
+  const int nnz = g.nnz;
+  int ku[6], kw[6];
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    ku[a] = c.kpt - 2 + a;
+    kw[a] = c.kwpt - 2 + a;
+  }
+  double wx[6], wy[6], wu[6], ww[6];
+  lag_horizontal(x, g.dx, c.ipt - 3, wx);
+  lag_horizontal(y, g.dy, c.jpt - 3, wy);
+  {
+    int lo = 0, hi = 5;  // of the six levels
+    if (c.kpt == 1) { lo = 2; hi = 3; ku[0] = 1; ku[1] = 1; }
+    else if (c.kpt == 0) { lo = 3; hi = 4; ku[0] = 1; ku[1] = 1; ku[2] = 1; }
+    else if (c.kpt < 0) { hi = -1; }
+    else if (c.kpt == 2) { lo = 1; hi = 4; }
+    else if (c.kpt == nnz) { lo = 1; hi = 2; ku[3] = nnz; ku[4] = nnz; ku[5] = nnz; }
+    else if (c.kpt > nnz) { hi = -1; }
+    else if (c.kpt == nnz - 1) { lo = 2; hi = 3; ku[4] = nnz; ku[5] = nnz; }
+    else if (c.kpt == nnz - 2) { lo = 1; hi = 4; }
+    lag_vertical(s_zz, ku, lo, hi, nnz + 1, z, wu);
+  }
+  {
+    int lo = 0, hi = 5;
+    if (c.kwpt == 0) { lo = 2; hi = 3; kw[0] = 1; kw[1] = 1; }
+    else if (c.kwpt < 0) { hi = -1; kw[0] = 1; kw[1] = 1; kw[2] = 1; }
+    else if (c.kwpt == 1) { lo = 1; hi = 4; kw[0] = 1; }
+    else if (c.kwpt == nnz - 1) { lo = 2; hi = 3; kw[4] = nnz; kw[5] = nnz; }
+    else if (c.kwpt >= nnz) { hi = -1; kw[2] = nnz; kw[3] = nnz; kw[4] = nnz; kw[5] = nnz; }
+    else if (c.kwpt == nnz - 2) { lo = 1; hi = 4; kw[5] = nnz; }
+    lag_vertical(s_z, kw, lo, hi, nnz + 1, z, ww);
+  }
+  const unsigned sj = (unsigned)F.sj, si = (unsigned)F.si;
+  unsigned ox[6], oy[6];
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    ox[a] = si * (unsigned)(clampi(c.ipt + a - 2, -1, g.nnx + 3) + 1);
+    oy[a] = sj * (unsigned)(clampi(c.jpt + a - 2, -1, g.nny + 3) + 1);
+  }
+  // the field's planes at levels b (weight w0) and b + 1 (w1)
+  auto planes = [&](const double* fld, unsigned b, double w0, double w1, double& sum) {
+    double hi[36];
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+#pragma unroll
       for (int i = 0; i < 6; ++i) {
-        const int ix = clampi(c.ipt + i - 2, -1, g.nnx + 3);
-        const int64_t o = ext_off(F, izuv, iy, ix), ow = ext_off(F, izw, iy, ix);
-        f.u[0] = f.u[0] + F.u[o] * wt[0][i] * wt[1][j] * wt[2][k];
-        f.u[1] = f.u[1] + F.v[o] * wt[0][i] * wt[1][j] * wt[2][k];
-        f.u[2] = f.u[2] + F.w[ow] * wt[0][i] * wt[1][j] * wt[3][k];
-        f.T = f.T + F.T[o] * wt[0][i] * wt[1][j] * wt[2][k];
-        f.q = f.q + F.q[o] * wt[0][i] * wt[1][j] * wt[2][k];
+        double lo;
+        node_pair(fld, ox[i] + oy[j] + b, lo, hi[6 * j + i]);
+        sum = sum + lo * wx[i] * wy[j] * w0;
       }
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+#pragma unroll
+      for (int i = 0; i < 6; ++i) sum = sum + hi[6 * j + i] * wx[i] * wy[j] * w1;
+    __builtin_amdgcn_sched_barrier(0);  // one field's planes in registers at a time
+  };
+  // Two of the six levels as b and b + 1.  Where the lists above repeat a level
+  // or step back, at most one of the entries that share a level has a weight,
+  // and levels further apart have none, so the weights move to their level.
+  auto pair_of = [&](const int k[6], const double w[6], double& w0, double& w1) {
+    const int a = clampi(k[0], 0, nnz + 1), d = clampi(k[1], 0, nnz + 1), b = min(min(a, d), nnz);
+    w0 = (a == b ? w[0] : 0.0) + (d == b ? w[1] : 0.0);
+    w1 = (a != b ? w[0] : 0.0) + (d != b ? w[1] : 0.0);
+    return (unsigned)b;
+  };
+  Fluid f = {{0.0, 0.0, 0.0}, 0.0, 0.0};
+#pragma unroll 1
+  for (int k = 0; k < 3; ++k) {
+    double u0, u1, w0, w1;
+    const unsigned bu = pair_of(ku, wu, u0, u1), bw = pair_of(kw, ww, w0, w1);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      ku[a] = ku[a + 2];
+      kw[a] = kw[a + 2];
+      wu[a] = wu[a + 2];
+      ww[a] = ww[a + 2];
     }
+    planes(F.u, bu, u0, u1, f.u[0]);
+    planes(F.v, bu, u0, u1, f.u[1]);
+    planes(F.w, bw, w0, w1, f.u[2]);
+    planes(F.T, bu, u0, u1, f.T);
+    planes(F.q, bu, u0, u1, f.q);
   }
   return f;
 }

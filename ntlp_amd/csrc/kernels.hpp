@@ -21,6 +21,13 @@
 
 namespace ntlp {
 
+// Waves per SIMD the register allocation of the droplet kernels must leave room
+// for: two with the 6th-order gather, whose planes of node values would
+// otherwise take a whole SIMD's registers for one wave (1090 instead of 930 us
+// for an FP64 step of 700k droplets); no bound else.
+template <int ILIN>
+constexpr int kMinWaves = ILIN == 1 ? 1 : 2;
+
 // hot column indices
 enum {
   kHX = 0, kHY, kHZ, kHVX, kHVY, kHVZ, kHTP, kHR, kHMS, kHKAPPA, kHRC, kHRES, kHACTRES, kHNUMACT, kNHot
@@ -409,7 +416,7 @@ __device__ __forceinline__ void count_key(int* counts, int key, bool valid) {
 // LAZY (BE steps of the library): the residence times stay in HBM until
 // k_res_settle at the end of the call.
 template <int MODE, int PREC, int ILIN, bool SERVE = false, bool LAZY = false>
-__global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
+__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
   const DevConsts& C = *a.Cp;
   extern __shared__ double s_dyn[];  // z(0:nnz+1) | zz(0:nnz+1) | field box (a.box_bytes)
   __shared__ int s_red[kTallyWidth + 1];
@@ -516,7 +523,7 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
 // particle_update_rk3(istage) / particle_update_BE in place on the current
 // buffers (no reordering), reading and writing the record columns.
 template <int MODE, int PREC, int ILIN>
-__global__ void __launch_bounds__(kBlock) k_update(StepArgs a) {
+__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_update(StepArgs a) {
   const DevConsts& C = *a.Cp;
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   __shared__ int s_red[kTallyWidth + 1];
@@ -551,7 +558,7 @@ __global__ void __launch_bounds__(kBlock) k_update(StepArgs a) {
 
 // uf_interp_lin / uf_interp for every droplet, optionally vp=uf and Tp=Tf.
 template <int ILIN>
-__global__ void __launch_bounds__(kBlock) k_interp(StepArgs a, int set_vp, int set_tp) {
+__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_interp(StepArgs a, int set_vp, int set_tp) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   const int64_t t = xcd_block() * kBlock + threadIdx.x;
   double x = 0.0, y = 0.0, z = 0.0;  // loaded before the barrier that follows the staging
@@ -1686,7 +1693,7 @@ struct AdmitArgs {
 };
 
 template <int ILIN>
-__global__ void __launch_bounds__(kBlock) k_serve_admit(AdmitArgs a) {
+__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_serve_admit(AdmitArgs a) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   stage_grid(a.g, s_z, s_zz);
   __syncthreads();
@@ -1763,7 +1770,7 @@ struct GenArgs {
 };
 
 template <int ILIN>
-__global__ void __launch_bounds__(kBlock) k_generate(GenArgs a) {
+__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_generate(GenArgs a) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   stage_grid(a.g, s_z, s_zz);
   __syncthreads();
