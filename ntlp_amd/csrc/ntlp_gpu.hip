@@ -387,6 +387,15 @@ void launch_scan(const int32_t* counts, int32_t* bsum, int32_t* offsets, int64_t
   }
 }
 
+// the counting sort of ctx.n keys whose counts are in place: perm lists their
+// indices by u cell, the counts are zero again
+int sort_keys(const int32_t* keys, const TallyClose* tc) {
+  CHK(launch("bin_scan", [&] { launch_scan(ctx.counts, ctx.bsum, ctx.offsets, ctx.ncell, tc, ctx.stream); }));
+  return launch("bin_scatter", [&] {
+    k_bin_scatter<<<bin_blocks(ctx.n), kBlock, 0, ctx.stream>>>(keys, ctx.n, ctx.offsets, ctx.counts, ctx.perm, nullptr);
+  });
+}
+
 // keys + counts of the current slot order must be in place; leaves perm
 // sorted by u cell (ties by `tie`, or by slot) and counts zeroed.  tc: closes
 // the counters of the step before on the way.
@@ -395,11 +404,7 @@ void launch_scan(const int32_t* counts, int32_t* bsum, int32_t* offsets, int64_t
 // atomics.  The fused step does not need that (a droplet's arithmetic does
 // not depend on its slot); the bin queries and the deterministic coupling do.
 int finish_bin(const int32_t* tie, bool canonical = true, const TallyClose* tc = nullptr) {
-  CHK(launch("bin_scan", [&] { launch_scan(ctx.counts, ctx.bsum, ctx.offsets, ctx.ncell, tc, ctx.stream); }));
-  CHK(launch("bin_scatter", [&] {
-    k_bin_scatter<<<bin_blocks(ctx.n), kBlock, 0, ctx.stream>>>(ctx.keys[ctx.cur], ctx.n, ctx.offsets, ctx.counts, ctx.perm,
-                                                              nullptr);
-  }));
+  CHK(sort_keys(ctx.keys[ctx.cur], tc));
   if (canonical)
     CHK(launch("bin_cellsort", [&] {
       k_cell_sort<<<grid_flat(ctx.ncell), kBlock, 0, ctx.stream>>>(ctx.offsets, ctx.ncell, ctx.perm, tie);
@@ -717,6 +722,7 @@ TallyClose next_close(bool be) {
 // caller needs the cold columns).
 // Steps between two reorderings of the slots into cell order.
 constexpr int kReorderEvery = 16;
+bool reorder_due() { return !ctx.slots_sorted || ctx.since_reorder + 1 >= kReorderEvery; }
 // Calls of fewer BE steps update the residence times in the step kernel: the
 // settle pass reads and writes the 32 bytes per droplet that a lazy step
 // saves, so it pays from about two steps on.
@@ -751,11 +757,12 @@ int empty_steps(int mode, int nsteps, bool scatter) {
 int run_fused_steps(int mode, int prec, int nsteps, int it0, bool scatter, bool lazy, int& done) {
   const unsigned mask = mode == NTLP_MODE_RK3 ? kDiagRK3 : kDiagBE;
   if (ctx.diag_mask & ~mask) CHK(flush_diag());
-  if (!ctx.perm_valid || !ctx.keys_valid) CHK(bin_current(nullptr, nullptr));
+  // the first step reads the keys, and the sort where it reorders the slots
+  if (!ctx.keys_valid || (!ctx.perm_valid && reorder_due())) CHK(bin_current(nullptr, nullptr));
   ctx.amounts_valid = false;
   ctx.amounts_f32 = prec == PREC_MIXED;  // the step kernels' amounts
   for (int k = 0; k < nsteps; ++k) {
-    const bool reorder = !ctx.slots_sorted || ctx.since_reorder + 1 >= kReorderEvery;
+    const bool reorder = reorder_due();
     StepArgs a = base_args();
     a.it = it0 + k;
     a.write_cold = (k == nsteps - 1) ? 1 : 0;
@@ -1323,15 +1330,29 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
   a.mult = ctx.mult[0];
   a.home = ctx.home[0];
   a.cold = ctx.cold;
+  a.diag = ctx.diag;
   a.pidx = ctx.pidx;
   a.procidx = ctx.procidx;
+  a.put_keys = ctx.keys[1];
+  a.keys = ctx.keys[0];
+  a.counts = ctx.counts;
+  a.perm = ctx.perm;
   const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
   const bool lin = ctx.fl.ilin == 1;
+  if (!rc) rc = launch("generate", [&] { k_gen_keys<<<grid, kBlock, 0, ctx.stream>>>(a); });
+  if (!rc) rc = sort_keys(ctx.keys[1], nullptr);
   if (!rc)
     rc = launch("generate", [&] {
-      if (lin) k_generate<1><<<grid, kBlock, 0, ctx.stream>>>(a);
-      else k_generate<0><<<grid, kBlock, 0, ctx.stream>>>(a);
+      if (lin) k_generate<1><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
+      else k_generate<0><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
     });
+  if (!rc) {  // slots in cell order with their keys; uf, Tf and qinf wait in diag
+    ctx.home_identity = false;
+    ctx.slots_sorted = true;
+    ctx.since_reorder = 0;
+    ctx.keys_valid = true;
+    ctx.diag_mask = (1u << kCUFX) | (1u << kCUFY) | (1u << kCUFZ) | (1u << kCTF) | (1u << kCQINF);
+  }
   if (hipStreamSynchronize(ctx.stream) != hipSuccess && !rc) rc = fail(NTLP_E_HIP, "ensemble generation failed");
   dfree(d_ens);
   dfree(d_start);
