@@ -340,6 +340,16 @@ __global__ void __launch_bounds__(kBlock) k_res_settle(double* hot, int64_t n, i
   }
 }
 
+// Where the record columns outside the hot state stand: the put-order columns,
+// read through home, or (home null) the slot-order ones that the last update
+// left.
+struct ColdView {
+  const double* base;
+  const int32_t* home;
+  int64_t cap;
+  __device__ __forceinline__ int64_t row(int64_t t) const { return home ? (int64_t)home[t] : t; }
+};
+
 __device__ __forceinline__ void load_rhs(const double* cold, int64_t cap, int64_t h, Diag& o) {
   o.xrhs[0] = cold[kCXRHSX * cap + h];
   o.xrhs[1] = cold[kCXRHSY * cap + h];
@@ -520,40 +530,48 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
 
 // ------------------------------------------------- reference entry points
 
-// particle_update_rk3(istage) / particle_update_BE in place on the current
-// buffers (no reordering), reading and writing the record columns.
-template <int MODE, int PREC, int ILIN>
-__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_update(StepArgs a) {
+// particle_update_rk3(istage) in place on the current buffers.  The stage
+// registers are read from `rhs` and the record columns written in slot order
+// (a.diag); put order is restored on demand.
+template <int PREC, int ILIN>
+__global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_update(StepArgs a, ColdView rhs) {
   const DevConsts& C = *a.Cp;
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
-  __shared__ int s_red[kTallyWidth + 1];
   const int64_t t = xcd_block() * kBlock + threadIdx.x;
-  Tally tl = {0, 0, 0, 0, 0, 0, 0, -1};
   // the droplet's loads go out before the barrier that follows the staging
   Drop d;
-  int32_t home = 0;
+  Diag o;
   if (t < a.n) {
     d = load_drop(a.src.hot, t);
-    home = a.src.home[t];
+    load_rhs(rhs.base, rhs.cap, rhs.row(t), o);
   }
   stage_grid(a.g, s_z, s_zz);
-  zero_tally_lds(s_red);
   __syncthreads();
-  if (t < a.n) {
-    Diag o;
-    if (MODE == 1) {
-      load_rhs(a.cold, a.cap, home, o);
-      rk3_droplet<PREC, ILIN>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.istage, a.it, o);
-      store_rhs(a.cold, a.cap, home, o);
-      if (a.istage == 1) store_old(a.cold, a.cap, home, o);
-    } else {
-      be_droplet<PREC, ILIN>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, -1, a.flux, a.src.mult[t]);
-      store_old(a.cold, a.cap, home, o);
-    }
-    store_gathered(a.cold, a.cap, home, o);
-    store_dynamic(a.src.hot, t, d);
-  }
-  if (MODE == 2) flush_tally(tl, a.tally, s_red);
+  if (t >= a.n) return;
+  rk3_droplet<PREC, ILIN>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.istage, a.it, o);
+  store_rhs(a.diag, a.cap, t, o);
+  if (a.istage == 1) store_old(a.diag, a.cap, t, o);
+  store_gathered(a.diag, a.cap, t, o);
+  store_dynamic(a.src.hot, t, d);
+}
+
+// The slots in cell order (perm): every column, mult, home and key of slot
+// perm[t] to slot t of the other buffers.
+__global__ void __launch_bounds__(kBlock) k_reorder(DropletBufs src, DropletBufs dst, const int32_t* perm,
+                                                    const int32_t* keys_in, int32_t* keys, int64_t n) {
+  const int64_t t = xcd_block() * kBlock + threadIdx.x;
+  if (t >= n) return;
+  const int64_t s = perm[t];
+  double v[kNHot];
+#pragma unroll
+  for (int c = 0; c < kNHot; ++c) v[c] = src.hot[hix(c, s)];
+  const int64_t mult = src.mult[s];
+  const int32_t home = src.home[s], key = keys_in[s];
+#pragma unroll
+  for (int c = 0; c < kNHot; ++c) dst.hot[hix(c, t)] = v[c];
+  dst.mult[t] = mult;
+  dst.home[t] = home;
+  keys[t] = key;
 }
 
 // uf_interp_lin / uf_interp for every droplet, optionally vp=uf and Tp=Tf.
@@ -573,12 +591,11 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_interp(StepArgs a, 
   const Cell c = cell_of(a.g, s_z, s_zz, x, y, z);
   Fluid f = (ILIN == 1) ? gather_lin_f64<true>(a.g, a.F, s_z, s_zz, x, y, z, c)
                         : gather6_f64(a.g, a.F, s_z, s_zz, x, y, z, c);
-  const int32_t h = a.src.home[t];
-  a.cold[kCUFX * a.cap + h] = f.u[0];
-  a.cold[kCUFY * a.cap + h] = f.u[1];
-  a.cold[kCUFZ * a.cap + h] = f.u[2];
-  a.cold[kCTF * a.cap + h] = f.T;
-  a.cold[kCQINF * a.cap + h] = f.q;
+  a.diag[kCUFX * a.cap + t] = f.u[0];  // slot order, like the steps' diagnostics
+  a.diag[kCUFY * a.cap + t] = f.u[1];
+  a.diag[kCUFZ * a.cap + t] = f.u[2];
+  a.diag[kCTF * a.cap + t] = f.T;
+  a.diag[kCQINF * a.cap + t] = f.q;
   if (set_vp) {
     a.src.hot[hix(kHVX, t)] = f.u[0];
     a.src.hot[hix(kHVY, t)] = f.u[1];
@@ -589,15 +606,15 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_interp(StepArgs a, 
 
 // Coupling amounts of the current state from the stored pre-step values
 // (particle_coupling_update's per-droplet part).
-__global__ void __launch_bounds__(kBlock) k_amounts(StepArgs a) {
+__global__ void __launch_bounds__(kBlock) k_amounts(StepArgs a, ColdView old) {
   const int64_t t = xcd_block() * kBlock + threadIdx.x;
   if (t >= a.n) return;
   const Drop d = load_drop(a.src.hot, t);
-  const int32_t h = a.src.home[t];
-  const double vold[3] = {a.cold[kCVXOLD * a.cap + h], a.cold[kCVYOLD * a.cap + h], a.cold[kCVZOLD * a.cap + h]};
+  const int64_t h = old.row(t), cap = old.cap;
+  const double vold[3] = {old.base[kCVXOLD * cap + h], old.base[kCVYOLD * cap + h], old.base[kCVZOLD * cap + h]};
   double am[6];
-  coupling_amounts(a.C, a.fl, d, a.cold[kCTF * a.cap + h], vold, a.cold[kCTPOLD * a.cap + h],
-                   a.cold[kCRADIUSOLD * a.cap + h], a.src.mult[t], am);
+  coupling_amounts(a.C, a.fl, d, old.base[kCTF * cap + h], vold, old.base[kCTPOLD * cap + h],
+                   old.base[kCRADIUSOLD * cap + h], a.src.mult[t], am);
 #pragma unroll
   for (int k = 0; k < 6; ++k) a.amounts[aix(k, t)] = am[k];
 }
@@ -1270,8 +1287,7 @@ struct StatsArgs {
   DevConsts C;
   const double* hot;
   const int64_t* mult;
-  const int32_t* home;
-  const double* cold;
+  ColdView cold;
   int64_t n, cap;
   int q0, nq;        // per-level quantities of this pass
   double* part0;     // [gridDim.x][kStats0] (pass 0 only)
@@ -1295,9 +1311,10 @@ __global__ void __launch_bounds__(kBlock) k_xy_stats(StatsArgs a) {
   const double pi = 4.0 * atan(1.0);
   for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
     const Drop d = load_drop(a.hot, t);
-    const int64_t h = a.home[t];
-    const double uf0 = a.cold[kCUFX * a.cap + h], uf1 = a.cold[kCUFY * a.cap + h], uf2 = a.cold[kCUFZ * a.cap + h];
-    const double Tf = a.cold[kCTF * a.cap + h], qinf = a.cold[kCQINF * a.cap + h];
+    const int64_t h = a.cold.row(t);
+    const double* cold = a.cold.base;
+    const double uf0 = cold[kCUFX * a.cap + h], uf1 = cold[kCUFY * a.cap + h], uf2 = cold[kCUFZ * a.cap + h];
+    const double Tf = cold[kCTF * a.cap + h], qinf = cold[kCQINF * a.cap + h];
     const double m = (double)a.mult[t];
     const double mw = a.C.rhow * 4.0 / 3.0 * pi * pow(d.r, 3);
     if (first) {
@@ -1325,7 +1342,7 @@ __global__ void __launch_bounds__(kBlock) k_xy_stats(StatsArgs a) {
     if (kc >= 0) {
       const double q[24] = {1.0, d.vx, d.vy, d.vz, d.vx * d.vx, d.vy * d.vy, d.vz * d.vz, d.vx * d.vz,
                             uf0, uf1, uf2, uf0 * uf0, uf1 * uf1, uf2 * uf2, d.Tp, d.Tp * d.Tp, Tf,
-                            d.r, d.r * d.r, qinf, d.Tp * d.vz, m, m * mw, a.cold[kCQSTAR * a.cap + h]};
+                            d.r, d.r * d.r, qinf, d.Tp * d.vz, m, m * mw, cold[kCQSTAR * a.cap + h]};
 #pragma unroll
       for (int k = 0; k < 24; ++k)
         if (k >= a.q0 && k < a.q0 + a.nq) atomicAdd(&s_lvl[(k - a.q0) * nz2 + kc], q[k]);

@@ -426,7 +426,7 @@ int canonical_perm() {
 }
 
 // bin the current slot order from the positions
-int bin_current(int32_t* cellidx_dev, const int32_t* tie) {
+int bin_current(int32_t* cellidx_dev, const int32_t* tie, bool canonical = true) {
   BinArgs b;
   b.g = ctx.g;
   b.hot = ctx.hot[ctx.cur];
@@ -437,7 +437,7 @@ int bin_current(int32_t* cellidx_dev, const int32_t* tie) {
   b.cellidx = cellidx_dev;
   CHK(launch("bin_keys", [&] { k_keys<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(b); }));
   ctx.keys_valid = true;
-  return finish_bin(tie);
+  return finish_bin(tie, canonical);
 }
 
 unsigned src_mask() {
@@ -528,7 +528,7 @@ int tile_sorted() {
 }
 
 int scatter_tile() {
-  if (!ctx.perm_valid || !ctx.keys_valid) CHK(bin_current(nullptr, nullptr));
+  if (!ctx.perm_valid || !ctx.keys_valid) CHK(bin_current(nullptr, nullptr, false));
   return tile_sorted();
 }
 
@@ -536,9 +536,13 @@ int scatter_tile() {
 constexpr unsigned kDiagBE = (1u << kCUFX) | (1u << kCUFY) | (1u << kCUFZ) | (1u << kCTF) | (1u << kCQINF) |
                              (1u << kCQSTAR) | (1u << kCVXOLD) | (1u << kCVYOLD) | (1u << kCVZOLD) |
                              (1u << kCTPOLD) | (1u << kCRADIUSOLD);
-constexpr unsigned kDiagRK3 = kDiagBE | (1u << kCXRHSX) | (1u << kCXRHSY) | (1u << kCXRHSZ) | (1u << kCVRHSX) |
-                              (1u << kCVRHSY) | (1u << kCVRHSZ) | (1u << kCTPRHS_S) | (1u << kCTPRHS_L) |
-                              (1u << kCRADRHS);
+constexpr unsigned kDiagRhs = (1u << kCXRHSX) | (1u << kCXRHSY) | (1u << kCXRHSZ) | (1u << kCVRHSX) | (1u << kCVRHSY) |
+                              (1u << kCVRHSZ) | (1u << kCTPRHS_S) | (1u << kCTPRHS_L) | (1u << kCRADRHS);
+constexpr unsigned kDiagRK3 = kDiagBE | kDiagRhs;
+// the fluid at the droplets, the same with q*, the values before the step
+constexpr unsigned kDiagFluid = (1u << kCUFX) | (1u << kCUFY) | (1u << kCUFZ) | (1u << kCTF) | (1u << kCQINF);
+constexpr unsigned kDiagStats = kDiagFluid | (1u << kCQSTAR);
+constexpr unsigned kDiagOld = (1u << kCVXOLD) | (1u << kCVYOLD) | (1u << kCVZOLD) | (1u << kCTPOLD) | (1u << kCRADIUSOLD);
 
 // puts the pending diagnostics into the put-order cold columns
 int flush_diag() {
@@ -551,6 +555,48 @@ int flush_diag() {
     k_flush_diag<<<grid_flat(ctx.n), kBlock, 0, ctx.stream>>>(diag, home, ctx.n, ctx.cap, mask, cold);
   }));
   ctx.diag_mask = 0;
+  return 0;
+}
+
+// the record columns `need`: in slot order if the last update left all of
+// them there, else in put order
+int cold_view(unsigned need, ColdView& v) {
+  if ((ctx.diag_mask & need) == need) {
+    v = {ctx.diag, nullptr, ctx.cap};
+    return 0;
+  }
+  CHK(flush_diag());
+  v = {ctx.cold, ctx.home[ctx.cur], ctx.cap};
+  return 0;
+}
+
+// Steps between two reorderings of the slots into cell order.
+constexpr int kReorderEvery = 16;
+bool reorder_due() { return !ctx.slots_sorted || ctx.since_reorder + 1 >= kReorderEvery; }
+
+// The slots in cell order, for updates that do not reorder by themselves: with
+// the droplets in put order every gather takes 20 cache lines of its own and
+// the record columns are read and written at random through home.  1.5M
+// droplets on 96x80x64: an RK3 stage 401 -> 143 us, the coupling scatter
+// after it 453 -> 119 us, for a reordering of 490 us after a put (less later).
+// Populations below kSortSlotsMin stay as they are: their sort is bound by its
+// launches.  The amounts of a step are lost (slot order).
+constexpr int64_t kSortSlotsMin = 8192;
+int sort_slots() {
+  if (!reorder_due() || ctx.n < kSortSlotsMin) return 0;
+  CHK(flush_diag());
+  if (!ctx.perm_valid || !ctx.keys_valid) CHK(bin_current(nullptr, nullptr, false));
+  const int c = ctx.cur, d = 1 - c;
+  const DropletBufs src = {ctx.hot[c], ctx.mult[c], ctx.home[c]}, dst = {ctx.hot[d], ctx.mult[d], ctx.home[d]};
+  CHK(launch("reorder", [&] {
+    k_reorder<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(src, dst, ctx.perm, ctx.keys[c], ctx.keys[d], ctx.n);
+  }));
+  ctx.cur = d;
+  ctx.home_identity = false;
+  ctx.slots_sorted = true;
+  ctx.since_reorder = 0;
+  ctx.perm_valid = false;  // perm sorted the old slots
+  ctx.amounts_valid = false;
   return 0;
 }
 
@@ -612,7 +658,7 @@ StatsShape stats_shape() {
 // and lw [nny][nnx] (all device memory).  timed: through launch() (HIP events
 // when timing is on); otherwise the kernels are launched directly, so that the
 // call creates nothing.
-int stats_launch(const StatsShape& sh, double* part0, double* part1, double* out0, double* out1, double* lw,
+int stats_launch(const StatsShape& sh, const ColdView& cold, double* part0, double* part1, double* out0, double* out1, double* lw,
                  bool timed) {
   auto go = [&](const char* name, auto&& f) -> int {
     if (timed) return launch(name, f);
@@ -628,8 +674,7 @@ int stats_launch(const StatsShape& sh, double* part0, double* part1, double* out
     a.C = ctx.C;
     a.hot = ctx.hot[ctx.cur];
     a.mult = ctx.mult[ctx.cur];
-    a.home = ctx.home[ctx.cur];
-    a.cold = ctx.cold;
+    a.cold = cold;
     a.n = ctx.n;
     a.cap = ctx.cap;
     a.q0 = q0;
@@ -650,9 +695,9 @@ int stats_launch(const StatsShape& sh, double* part0, double* part1, double* out
   return 0;
 }
 
-template <int MODE, int PREC, int ILIN>
-void launch_update_t(const StepArgs& a, unsigned grid) {
-  k_update<MODE, PREC, ILIN><<<grid, kBlock, 0, ctx.stream>>>(a);
+template <int PREC, int ILIN>
+void launch_update_t(const StepArgs& a, const ColdView& rhs, unsigned grid) {
+  k_update<PREC, ILIN><<<grid, kBlock, 0, ctx.stream>>>(a, rhs);
 }
 template <int MODE, int PREC, int ILIN>
 void launch_step_t(const StepArgs& a, unsigned grid, bool lazy) {
@@ -666,15 +711,13 @@ void launch_step_t(const StepArgs& a, unsigned grid, bool lazy) {
   k_step<MODE, PREC, ILIN><<<grid, kBlock, lds, ctx.stream>>>(a);
 }
 
-template <int MODE>
-int dispatch_update(const StepArgs& a, int prec) {
+int dispatch_update(const StepArgs& a, const ColdView& rhs, int prec) {
   const unsigned gr = grid8(a.n);
   const bool lin = ctx.fl.ilin == 1;
-  const char* name = MODE == 1 ? "update_rk3" : "update_be";
-  return launch(name, [&] {
-    if (prec == PREC_FP64) lin ? launch_update_t<MODE, 0, 1>(a, gr) : launch_update_t<MODE, 0, 0>(a, gr);
-    else if (prec == PREC_MIXED) lin ? launch_update_t<MODE, 1, 1>(a, gr) : launch_update_t<MODE, 1, 0>(a, gr);
-    else lin ? launch_update_t<MODE, 2, 1>(a, gr) : launch_update_t<MODE, 2, 0>(a, gr);
+  return launch("update_rk3", [&] {
+    if (prec == PREC_FP64) lin ? launch_update_t<0, 1>(a, rhs, gr) : launch_update_t<0, 0>(a, rhs, gr);
+    else if (prec == PREC_MIXED) lin ? launch_update_t<1, 1>(a, rhs, gr) : launch_update_t<1, 0>(a, rhs, gr);
+    else lin ? launch_update_t<2, 1>(a, rhs, gr) : launch_update_t<2, 0>(a, rhs, gr);
   });
 }
 
@@ -720,9 +763,6 @@ TallyClose next_close(bool be) {
 // then sorts for the next step and (scatter) deposits the sources.  The last
 // step leaves its diagnostics in slot order (put order is restored when a
 // caller needs the cold columns).
-// Steps between two reorderings of the slots into cell order.
-constexpr int kReorderEvery = 16;
-bool reorder_due() { return !ctx.slots_sorted || ctx.since_reorder + 1 >= kReorderEvery; }
 // Calls of fewer BE steps update the residence times in the step kernel: the
 // settle pass reads and writes the 32 bytes per droplet that a lazy step
 // saves, so it pays from about two steps on.
@@ -758,7 +798,7 @@ int run_fused_steps(int mode, int prec, int nsteps, int it0, bool scatter, bool 
   const unsigned mask = mode == NTLP_MODE_RK3 ? kDiagRK3 : kDiagBE;
   if (ctx.diag_mask & ~mask) CHK(flush_diag());
   // the first step reads the keys, and the sort where it reorders the slots
-  if (!ctx.keys_valid || (!ctx.perm_valid && reorder_due())) CHK(bin_current(nullptr, nullptr));
+  if (!ctx.keys_valid || (!ctx.perm_valid && reorder_due())) CHK(bin_current(nullptr, nullptr, false));
   ctx.amounts_valid = false;
   ctx.amounts_f32 = prec == PREC_MIXED;  // the step kernels' amounts
   for (int k = 0; k < nsteps; ++k) {
@@ -1351,7 +1391,7 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
     ctx.slots_sorted = true;
     ctx.since_reorder = 0;
     ctx.keys_valid = true;
-    ctx.diag_mask = (1u << kCUFX) | (1u << kCUFY) | (1u << kCUFZ) | (1u << kCTF) | (1u << kCQINF);
+    ctx.diag_mask = kDiagFluid;
   }
   if (hipStreamSynchronize(ctx.stream) != hipSuccess && !rc) rc = fail(NTLP_E_HIP, "ensemble generation failed");
   dfree(d_ens);
@@ -1395,14 +1435,17 @@ int ntlp_gpu_crit_radius(void) {
 int ntlp_gpu_interp(int32_t set_vp, int32_t set_tp) {
   CHK(need_drops());
   if (ctx.n == 0) return NTLP_OK;
-  CHK(flush_diag());
-  if (set_vp || set_tp) ctx.amounts_valid = false;
+  if (set_vp || set_tp) {  // the set-up of droplets that are stepped next
+    ctx.amounts_valid = false;
+    CHK(sort_slots());
+  }
   StepArgs a = base_args();
   const bool lin = ctx.fl.ilin == 1;
   CHK(launch("interp", [&] {
     if (lin) k_interp<1><<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(a, set_vp, set_tp);
     else k_interp<0><<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(a, set_vp, set_tp);
   }));
+  ctx.diag_mask |= kDiagFluid;
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
@@ -1417,13 +1460,18 @@ int ntlp_gpu_particle_update_rk3_prec(int32_t istage, int32_t it, int32_t prec) 
   CHK(check_prec(prec));
   if (istage < 1 || istage > 3) return fail(NTLP_E_INVALID, "istage must be 1, 2 or 3");
   if (ctx.n == 0) return NTLP_OK;
-  CHK(flush_diag());
+  if (istage == 1 || !ctx.slots_sorted) CHK(sort_slots());
+  if (istage == 1) ctx.since_reorder++;
   ctx.keys_valid = false;
   ctx.amounts_valid = false;
   StepArgs a = base_args();
   a.istage = istage;
   a.it = it;
-  CHK(dispatch_update<1>(a, prec));
+  // the stage registers of the stage before; put-order ones after a put
+  ColdView rhs = {ctx.diag, nullptr, ctx.cap};
+  if ((ctx.diag_mask & kDiagRhs) != kDiagRhs) rhs = {ctx.cold, ctx.home[ctx.cur], ctx.cap};
+  CHK(dispatch_update(a, rhs, prec));
+  ctx.diag_mask |= kDiagRhs | kDiagStats | (istage == 1 ? kDiagOld : 0u);
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
@@ -1458,9 +1506,10 @@ int ntlp_gpu_particle_coupling_update(double* src_out, int32_t deterministic) {
     return NTLP_OK;
   }
   if (!ctx.amounts_valid) {  // amounts from the state and its old values in cold
-    CHK(flush_diag());
+    ColdView old;
+    CHK(cold_view(kDiagOld | (1u << kCTF), old));
     StepArgs a = base_args();
-    CHK(launch("amounts", [&] { k_amounts<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(a); }));
+    CHK(launch("amounts", [&] { k_amounts<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(a, old); }));
     ctx.amounts_valid = true;
     ctx.amounts_f32 = false;
   }
@@ -1668,7 +1717,8 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
 
 int ntlp_gpu_particle_xy_stats(double* s0, double* s1, double* lwp) {
   CHK(need_drops());
-  CHK(flush_diag());
+  ColdView cold;
+  CHK(cold_view(kDiagStats, cold));
   const StatsShape sh = stats_shape();
   double *part0 = nullptr, *part1 = nullptr, *out0 = nullptr, *out1 = nullptr, *lw = nullptr;
   int rc = dalloc(part0, (int64_t)sh.rows * kStats0, "statistics rows");
@@ -1676,7 +1726,7 @@ int ntlp_gpu_particle_xy_stats(double* s0, double* s1, double* lwp) {
   if (!rc) rc = dalloc(out0, kStats0, "statistics");
   if (!rc) rc = dalloc(out1, 24 * sh.nz2, "statistics");
   if (!rc) rc = dalloc(lw, (int64_t)ctx.g.nnx * ctx.g.nny, "LWP");
-  if (!rc) rc = stats_launch(sh, part0, part1, out0, out1, lw, true);
+  if (!rc) rc = stats_launch(sh, cold, part0, part1, out0, out1, lw, true);
   if (!rc && ((s0 && hipMemcpyAsync(s0, out0, sizeof(double) * kStats0, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess) ||
               (s1 && hipMemcpyAsync(s1, out1, sizeof(double) * 24 * sh.nz2, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess) ||
               (lwp && hipMemcpyAsync(lwp, lw, sizeof(double) * ctx.g.nnx * ctx.g.nny, hipMemcpyDeviceToHost,
@@ -1701,13 +1751,17 @@ int ntlp_gpu_particle_xy_stats_noalloc(double* s0, double* s1, double* lwp) {
   if (need > kStatsScratch)
     return fail(NTLP_E_RANGE, "statistics rows need " + std::to_string(need * 8) + " bytes of workspace; the static "
                 "workspace holds " + std::to_string(kStatsScratch * 8));
-  if (ctx.diag_mask) {  // pending diagnostics (uf, Tf, qinf, qstar) into the put-order columns
-    k_flush_diag<<<grid_flat(ctx.n), kBlock, 0, ctx.stream>>>(ctx.diag, ctx.home[ctx.cur], ctx.n, ctx.cap,
-                                                              ctx.diag_mask, ctx.cold);
-    HIPCHK(hipGetLastError());
-    ctx.diag_mask = 0;
+  ColdView cold = {ctx.diag, nullptr, ctx.cap};
+  if ((ctx.diag_mask & kDiagStats) != kDiagStats) {
+    if (ctx.diag_mask) {  // some of uf, Tf, qinf, qstar in slot order only: into the put-order columns
+      k_flush_diag<<<grid_flat(ctx.n), kBlock, 0, ctx.stream>>>(ctx.diag, ctx.home[ctx.cur], ctx.n, ctx.cap,
+                                                                ctx.diag_mask, ctx.cold);
+      HIPCHK(hipGetLastError());
+      ctx.diag_mask = 0;
+    }
+    cold = {ctx.cold, ctx.home[ctx.cur], ctx.cap};
   }
-  return stats_launch(sh, ws, ws + (int64_t)sh.rows * kStats0, s0, s1, lwp, false);
+  return stats_launch(sh, cold, ws, ws + (int64_t)sh.rows * kStats0, s0, s1, lwp, false);
 }
 
 int64_t ntlp_gpu_num_ucells(void) { return ctx.init ? ctx.ncell : 0; }
