@@ -1600,8 +1600,9 @@ __global__ void k_iota(int32_t* p, int64_t n) {
 }
 
 // Halo fill of fill_ext on one periodic domain: ext(k, j, i) for
-// j in -1..nny+3, i in -1..nnx+3 from core(k, 1..nny, 1..nnx).
-__global__ void k_fill_ext(const double* core, double* ext, int nnx, int nny, int nnz) {
+// j in -1..nny+3, i in -1..nnx+3 from core(k, 1..nny, 1..nnx); f32 (may be
+// null) receives the FP32 copy.
+__global__ void k_fill_ext(const double* core, double* ext, float* f32, int nnx, int nny, int nnz) {
   const int64_t nz2 = nnz + 2;
   const int64_t total = nz2 * (nny + 5) * (int64_t)(nnx + 5);
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
@@ -1611,13 +1612,15 @@ __global__ void k_fill_ext(const double* core, double* ext, int nnx, int nny, in
     const int i = (int)(r / (nny + 5)) - 1;
     const int jc = ((j - 1) % nny + nny) % nny + 1;
     const int ic = ((i - 1) % nnx + nnx) % nnx + 1;
-    ext[e] = core[k + nz2 * ((jc - 1) + (int64_t)nny * (ic - 1))];
+    const double v = core[k + nz2 * ((jc - 1) + (int64_t)nny * (ic - 1))];
+    ext[e] = v;
+    if (f32) f32[e] = (float)v;
   }
 }
 
 // xtoz_trans + fill_ext from the flow solver's x-fastest array
 // u(1:nnx+2, 1:nny, 0:nnz+1) (les.F:8394-8397, 10060-10131) to ext layout.
-__global__ void k_xpencil_to_ext(const double* xp, double* ext, int nnx, int nny, int nnz) {
+__global__ void k_xpencil_to_ext(const double* xp, double* ext, float* f32, int nnx, int nny, int nnz) {
   const int64_t nz2 = nnz + 2;
   const int64_t total = nz2 * (nny + 5) * (int64_t)(nnx + 5);
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
@@ -1627,7 +1630,9 @@ __global__ void k_xpencil_to_ext(const double* xp, double* ext, int nnx, int nny
     const int i = (int)(r / (nny + 5)) - 1;
     const int jc = ((j - 1) % nny + nny) % nny + 1;
     const int ic = ((i - 1) % nnx + nnx) % nnx + 1;
-    ext[e] = xp[(ic - 1) + (int64_t)(nnx + 2) * ((jc - 1) + (int64_t)nny * k)];
+    const double v = xp[(ic - 1) + (int64_t)(nnx + 2) * ((jc - 1) + (int64_t)nny * k)];
+    ext[e] = v;
+    if (f32) f32[e] = (float)v;
   }
 }
 
@@ -1869,11 +1874,100 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_generate(GenArgs a)
   a.diag[kCQINF * a.cap + t] = f.q;
 }
 
-// a plain column into hot column c (slot order)
-__global__ void k_pack_hot(const double* col, int c, int64_t n, double* hot) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) hot[hix(c, t)] = col[t];
+// Where a record column lives: hot column, cold column, or (both negative) nowhere.
+struct ColumnPlace {
+  int8_t hot[48], cold[48];  // by record column (or record word, k_records_*)
+};
+
+// Columns c0.. (blockIdx.y) of a put, n values each, to their places.
+__global__ void __launch_bounds__(kBlock) k_columns_in(const double* cols, int c0, ColumnPlace pl, int64_t n, int64_t cap,
+                                                       double* hot, double* cold) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int c = c0 + blockIdx.y;
+  const double v = cols[(int64_t)blockIdx.y * n + i];
+  if (pl.hot[c] >= 0) hot[hix(pl.hot[c], i)] = v;
+  else cold[pl.cold[c] * cap + i] = v;
 }
+
+// and of a get, in put order (home null: slot order is put order).
+__global__ void __launch_bounds__(kBlock) k_columns_out(double* cols, int c0, ColumnPlace pl, int64_t n, int64_t cap,
+                                                        const double* hot, const double* cold, const int32_t* home) {
+  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (t >= n) return;
+  const int c = c0 + blockIdx.y;
+  double* out = cols + (int64_t)blockIdx.y * n;
+  if (pl.hot[c] >= 0) out[home ? home[t] : t] = hot[hix(pl.hot[c], t)];
+  else out[t] = cold[pl.cold[c] * cap + t];
+}
+
+// Restart records: 352 bytes of `type particle` in the ifort layout
+// (particles.f90:76-85, 1929-1950), taken as 44 words of 8 bytes: four int32
+// (pidx, procidx, nbr_pidx, nbr_procidx), 39 reals, mult, two pointer slots.
+// A workgroup turns 64 records through LDS, so that both the records and the
+// columns move in whole cache lines (done word by word on one host thread,
+// 250k records took 20 ms each way).  i0: the put index of the chunk's first
+// record.
+constexpr int kRecWords = 44, kRecMult = 41, kRecTile = 64;
+
+__global__ void __launch_bounds__(kBlock) k_records_in(const uint64_t* rec, int64_t i0, int64_t m, ColumnPlace pl,
+                                                       int64_t cap, double* hot, double* cold, int64_t* mult,
+                                                       int32_t* pidx, int32_t* procidx) {
+  __shared__ uint64_t tile[kRecTile * (kRecWords + 1)];
+  const int64_t r0 = (int64_t)blockIdx.x * kRecTile;
+  const int rows = (int)min((int64_t)kRecTile, m - r0);
+  for (int e = threadIdx.x; e < rows * kRecWords; e += kBlock)
+    tile[e / kRecWords * (kRecWords + 1) + e % kRecWords] = rec[r0 * kRecWords + e];
+  __syncthreads();
+  const int row = threadIdx.x % kRecTile;
+  if (row >= rows) return;
+  const int64_t i = i0 + r0 + row;
+  for (int w = threadIdx.x / kRecTile; w < kRecWords; w += kBlock / kRecTile) {
+    const uint64_t v = tile[row * (kRecWords + 1) + w];
+    if (w == 0) {
+      pidx[i] = (int32_t)(uint32_t)v;
+      procidx[i] = (int32_t)(uint32_t)(v >> 32);
+    } else if (w == kRecMult) {
+      mult[i] = (int64_t)v;
+    } else if (pl.hot[w] >= 0) {
+      hot[hix(pl.hot[w], i)] = __longlong_as_double((long long)v);
+    } else if (pl.cold[w] >= 0) {
+      cold[pl.cold[w] * cap + i] = __longlong_as_double((long long)v);
+    }
+  }
+}
+
+// slot: put index -> slot (null: the same)
+__global__ void __launch_bounds__(kBlock) k_records_out(uint64_t* rec, int64_t i0, int64_t m, ColumnPlace pl, int64_t cap,
+                                                        const double* hot, const double* cold, const int64_t* mult,
+                                                        const int32_t* pidx, const int32_t* procidx,
+                                                        const int32_t* slot) {
+  __shared__ uint64_t tile[kRecTile * (kRecWords + 1)];
+  const int64_t r0 = (int64_t)blockIdx.x * kRecTile;
+  const int rows = (int)min((int64_t)kRecTile, m - r0);
+  const int row = threadIdx.x % kRecTile;
+  if (row < rows) {
+    const int64_t i = i0 + r0 + row, t = slot ? (int64_t)slot[i] : i;
+    for (int w = threadIdx.x / kRecTile; w < kRecWords; w += kBlock / kRecTile) {
+      uint64_t v = 0;
+      if (w == 0) v = (uint64_t)(uint32_t)pidx[i] | ((uint64_t)(uint32_t)procidx[i] << 32);
+      else if (w == 1) v = ~0ull;  // nbr_pidx, nbr_procidx = -1
+      else if (w == kRecMult) v = (uint64_t)mult[t];
+      else if (pl.hot[w] >= 0) v = (uint64_t)__double_as_longlong(hot[hix(pl.hot[w], t)]);
+      else if (pl.cold[w] >= 0) v = (uint64_t)__double_as_longlong(cold[pl.cold[w] * cap + i]);
+      tile[row * (kRecWords + 1) + w] = v;
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < rows * kRecWords; e += kBlock)
+    rec[r0 * kRecWords + e] = tile[e / kRecWords * (kRecWords + 1) + e % kRecWords];
+}
+
+__global__ void k_invert(const int32_t* home, int64_t n, int32_t* slot) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) slot[home[t]] = (int32_t)t;
+}
+
 // hot column c -> put order (home == nullptr: slot order is put order)
 __global__ void k_unpack_hot(const double* hot, int c, const int32_t* home, int64_t n, double* out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -57,7 +57,8 @@ struct Ctx {
   // fields
   double* ext[5] = {};
   float* f32[3] = {};
-  double* field_stage = nullptr;
+  double* xfer = nullptr;  // staging of host transfers (see xfer_stage)
+  int64_t xfer_cap = 0;    // its doubles
   bool have_fields = false;
   int64_t ext_elems = 0;
   // droplets
@@ -165,6 +166,15 @@ int cold_of(int c) {
   }
 }
 
+ColumnPlace column_places() {
+  ColumnPlace pl;
+  for (int c = 0; c < 48; ++c) {
+    pl.hot[c] = (int8_t)(c < NTLP_NREAL ? hot_of(c) : -1);
+    pl.cold[c] = (int8_t)(c < NTLP_NREAL ? cold_of(c) : -1);
+  }
+  return pl;
+}
+
 template <typename T>
 void dfree(T*& p) {
   if (p) (void)hipFree(p);
@@ -261,10 +271,25 @@ int fill_i32(int32_t* p, int64_t n, int32_t v) {
   return launch("fill", [&] { k_fill_i32<<<grid_flat(n), kBlock, 0, ctx.stream>>>(p, n, v); });
 }
 
+// The staging buffer with room for at least `least` doubles, `want` if that
+// stays below kXferBytes.  It is kept until the context is released: allocated
+// and freed on each call it cost 40 to 260 us.  Its users leave it to the next
+// in stream order.
+constexpr int64_t kXferBytes = 128ll << 20;
+int xfer_stage(int64_t least, int64_t want) {
+  const int64_t room = std::max(least, std::min<int64_t>(want, kXferBytes / 8));
+  if (room <= ctx.xfer_cap) return 0;
+  HIPCHK(hipStreamSynchronize(ctx.stream));
+  ctx.xfer_cap = 0;
+  CHK(dalloc(ctx.xfer, room, "transfer staging"));
+  ctx.xfer_cap = room;
+  return 0;
+}
+
 void release_all() {
   for (auto& p : ctx.ext) dfree(p);
   for (auto& p : ctx.f32) dfree(p);
-  dfree(ctx.field_stage);
+  dfree(ctx.xfer);
   for (int b = 0; b < 2; ++b) {
     dfree(ctx.hot[b]);
     dfree(ctx.mult[b]);
@@ -1034,29 +1059,24 @@ int ntlp_gpu_set_fields(const double* u, const double* v, const double* w, const
     if (!ctx.ext[f]) CHK(dalloc(ctx.ext[f], ctx.ext_elems, "ext field"));
   for (int f = 0; f < 3; ++f)
     if (!ctx.f32[f]) CHK(dalloc(ctx.f32[f], ctx.ext_elems, "fp32 field copy"));
-  if (layout != NTLP_LAYOUT_EXT && !ctx.field_stage) CHK(dalloc(ctx.field_stage, in_elems, "field staging"));
+  if (layout != NTLP_LAYOUT_EXT) CHK(xfer_stage(in_elems, in_elems));
+  // one staging buffer serves the fields in turn, in stream order
   for (int f = 0; f < 5; ++f) {
+    double* dst = ctx.ext[f];
+    float* o = f < 3 ? ctx.f32[f] : nullptr;
     if (layout == NTLP_LAYOUT_EXT) {
-      HIPCHK(hipMemcpyAsync(ctx.ext[f], in[f], sizeof(double) * in_elems, hipMemcpyHostToDevice, ctx.stream));
-    } else {
-      HIPCHK(hipMemcpyAsync(ctx.field_stage, in[f], sizeof(double) * in_elems, hipMemcpyHostToDevice, ctx.stream));
-      double* dst = ctx.ext[f];
-      const double* stg = ctx.field_stage;
-      if (layout == NTLP_LAYOUT_CORE)
-        CHK(launch("fill_ext", [&] { k_fill_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, nx, ny, nz); }));
-      else
-        CHK(launch("fill_ext", [&] {
-          k_xpencil_to_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, nx, ny, nz);
-        }));
+      HIPCHK(hipMemcpyAsync(dst, in[f], sizeof(double) * in_elems, hipMemcpyHostToDevice, ctx.stream));
+      if (o) CHK(launch("to_f32", [&] { k_to_f32<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(dst, o, ctx.ext_elems); }));
+      continue;
     }
-    if (f < 3) {
-      double* s = ctx.ext[f];
-      float* o = ctx.f32[f];
-      CHK(launch("to_f32", [&] { k_to_f32<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(s, o, ctx.ext_elems); }));
-    }
-    HIPCHK(hipStreamSynchronize(ctx.stream));  // staging buffer reuse
+    HIPCHK(hipMemcpyAsync(ctx.xfer, in[f], sizeof(double) * in_elems, hipMemcpyHostToDevice, ctx.stream));
+    const double* stg = ctx.xfer;
+    CHK(launch("fill_ext", [&] {
+      if (layout == NTLP_LAYOUT_CORE) k_fill_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, o, nx, ny, nz);
+      else k_xpencil_to_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, o, nx, ny, nz);
+    }));
   }
-  dfree(ctx.field_stage);
+  HIPCHK(hipStreamSynchronize(ctx.stream));  // the host arrays are the caller's again
   ctx.have_fields = true;
   return NTLP_OK;
 }
@@ -1148,18 +1168,17 @@ int ntlp_gpu_particles_put(const double* soa, const int64_t* mult, const int32_t
   if (n >= (int64_t)INT32_MAX) return fail(NTLP_E_RANGE, "more than 2^31-1 droplets");
   CHK(ensure_capacity(n));
   if (n == 0) return NTLP_OK;
-  for (int c = 0; c < NTLP_NREAL; ++c) {
-    if (hot_of(c) >= 0) {
-      double* tmp = ctx.col_tmp;
-      double* hot = ctx.hot[0];
-      const int hc = hot_of(c);
-      HIPCHK(hipMemcpyAsync(tmp, soa + (int64_t)c * n, sizeof(double) * n, hipMemcpyHostToDevice, ctx.stream));
-      CHK(launch("put", [&] { k_pack_hot<<<grid_flat(n), kBlock, 0, ctx.stream>>>(tmp, hc, n, hot); }));
-      HIPCHK(hipStreamSynchronize(ctx.stream));  // col_tmp reuse
-    } else {
-      HIPCHK(hipMemcpyAsync(ctx.cold + (int64_t)cold_of(c) * ctx.cap, soa + (int64_t)c * n, sizeof(double) * n,
-                            hipMemcpyHostToDevice, ctx.stream));
-    }
+  // as many columns at a time as the staging buffer holds
+  CHK(xfer_stage(n, NTLP_NREAL * n));
+  const int per = (int)std::min<int64_t>(NTLP_NREAL, ctx.xfer_cap / n);
+  const ColumnPlace pl = column_places();
+  for (int c = 0; c < NTLP_NREAL; c += per) {
+    const int nc = std::min(per, NTLP_NREAL - c);
+    HIPCHK(hipMemcpyAsync(ctx.xfer, soa + (int64_t)c * n, sizeof(double) * nc * n, hipMemcpyHostToDevice, ctx.stream));
+    CHK(launch("put", [&] {
+      k_columns_in<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(ctx.xfer, c, pl, n, ctx.cap,
+                                                                                              ctx.hot[0], ctx.cold);
+    }));
   }
   HIPCHK(hipMemcpyAsync(ctx.mult[0], mult, sizeof(int64_t) * n, hipMemcpyHostToDevice, ctx.stream));
   if (pidx) HIPCHK(hipMemcpyAsync(ctx.pidx, pidx, sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx.stream));
@@ -1178,22 +1197,19 @@ int ntlp_gpu_particles_get(double* soa, int64_t* mult, int32_t* pidx, int32_t* p
     return fail(NTLP_E_STATE, "a failed step call left the droplets inconsistent: put them again");
   if (soa) CHK(flush_diag());
   if (n == 0) return NTLP_OK;
-  const int64_t cap = ctx.cap;
   const int32_t* home = ctx.home[ctx.cur];
   if (soa) {
-    for (int c = 0; c < NTLP_NREAL; ++c) {
-      if (hot_of(c) >= 0) {
-        const double* hot = ctx.hot[ctx.cur];
-        const int hc = hot_of(c);
-        double* tmp = ctx.col_tmp;
-        const int32_t* hm = ctx.home_identity ? nullptr : home;
-        CHK(launch("get", [&] { k_unpack_hot<<<grid_flat(n), kBlock, 0, ctx.stream>>>(hot, hc, hm, n, tmp); }));
-        HIPCHK(hipMemcpyAsync(soa + (int64_t)c * n, tmp, sizeof(double) * n, hipMemcpyDeviceToHost, ctx.stream));
-        HIPCHK(hipStreamSynchronize(ctx.stream));  // col_tmp reuse
-      } else {
-        HIPCHK(hipMemcpyAsync(soa + (int64_t)c * n, ctx.cold + (int64_t)cold_of(c) * cap, sizeof(double) * n,
-                              hipMemcpyDeviceToHost, ctx.stream));
-      }
+    CHK(xfer_stage(n, NTLP_NREAL * n));
+    const int per = (int)std::min<int64_t>(NTLP_NREAL, ctx.xfer_cap / n);
+    const ColumnPlace pl = column_places();
+    const int32_t* hm = ctx.home_identity ? nullptr : home;
+    for (int c = 0; c < NTLP_NREAL; c += per) {
+      const int nc = std::min(per, NTLP_NREAL - c);
+      CHK(launch("get", [&] {
+        k_columns_out<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(
+            ctx.xfer, c, pl, n, ctx.cap, ctx.hot[ctx.cur], ctx.cold, hm);
+      }));
+      HIPCHK(hipMemcpyAsync(soa + (int64_t)c * n, ctx.xfer, sizeof(double) * nc * n, hipMemcpyDeviceToHost, ctx.stream));
     }
   }
   if (mult) {
@@ -1204,7 +1220,6 @@ int ntlp_gpu_particles_get(double* soa, int64_t* mult, int32_t* pidx, int32_t* p
       col = tmp;
     }
     HIPCHK(hipMemcpyAsync(mult, col, sizeof(int64_t) * n, hipMemcpyDeviceToHost, ctx.stream));
-    HIPCHK(hipStreamSynchronize(ctx.stream));
   }
   if (pidx) HIPCHK(hipMemcpyAsync(pidx, ctx.pidx, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx.stream));
   if (procidx) HIPCHK(hipMemcpyAsync(procidx, ctx.procidx, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx.stream));
@@ -1227,45 +1242,68 @@ const int kRecCol[kRecReals] = {
     -1, -1, -1 /*u_sub*/, -1 /*sigm_s*/, NTLP_VXOLD, NTLP_VYOLD, NTLP_VZOLD, NTLP_TPOLD, NTLP_RADIUSOLD};
 }  // namespace
 
+// places of the record's 44 words
+static ColumnPlace record_places() {
+  ColumnPlace pl;
+  for (int w = 0; w < 48; ++w) {
+    const int c = (w >= 2 && w < 2 + kRecReals) ? kRecCol[w - 2] : -1;
+    pl.hot[w] = (int8_t)(c >= 0 ? hot_of(c) : -1);
+    pl.cold[w] = (int8_t)(c >= 0 ? cold_of(c) : -1);
+  }
+  return pl;
+}
+
 int ntlp_gpu_particles_put_records(const void* records, int64_t n) {
   if (n < 0 || (n > 0 && !records)) return fail(NTLP_E_INVALID, "bad record buffer");
-  std::vector<double> soa((size_t)n * NTLP_NREAL, 0.0);
-  std::vector<int64_t> mult((size_t)n);
-  std::vector<int32_t> pidx((size_t)n), procidx((size_t)n);
+  CHK(need_init());
+  if (n >= (int64_t)INT32_MAX) return fail(NTLP_E_RANGE, "more than 2^31-1 droplets");
+  CHK(ensure_capacity(n));
+  if (n == 0) return NTLP_OK;
+  CHK(xfer_stage(kRecWords, kRecWords * n));
+  const int64_t per = std::min(n, ctx.xfer_cap / kRecWords);
+  const ColumnPlace pl = record_places();
   const unsigned char* base = (const unsigned char*)records;
-  for (int64_t i = 0; i < n; ++i) {
-    const unsigned char* r = base + i * NTLP_RECORD_BYTES;
-    int32_t ints[4];
-    double reals[kRecReals];
-    memcpy(ints, r, 16);
-    memcpy(reals, r + 16, 8 * kRecReals);
-    memcpy(&mult[i], r + 16 + 8 * kRecReals, 8);
-    pidx[i] = ints[0];
-    procidx[i] = ints[1];
-    for (int k = 0; k < kRecReals; ++k)
-      if (kRecCol[k] >= 0) soa[(size_t)kRecCol[k] * n + i] = reals[k];
+  for (int64_t i = 0; i < n; i += per) {
+    const int64_t m = std::min(per, n - i);
+    HIPCHK(hipMemcpyAsync(ctx.xfer, base + i * NTLP_RECORD_BYTES, (size_t)m * NTLP_RECORD_BYTES, hipMemcpyHostToDevice,
+                          ctx.stream));
+    CHK(launch("put", [&] {
+      k_records_in<<<(unsigned)((m + kRecTile - 1) / kRecTile), kBlock, 0, ctx.stream>>>(
+          (const uint64_t*)ctx.xfer, i, m, pl, ctx.cap, ctx.hot[0], ctx.cold, ctx.mult[0], ctx.pidx, ctx.procidx);
+    }));
   }
-  return ntlp_gpu_particles_put(soa.data(), mult.data(), pidx.data(), procidx.data(), n);
+  CHK(launch("iota", [&] { k_iota<<<grid_flat(n), kBlock, 0, ctx.stream>>>(ctx.home[0], n); }));
+  HIPCHK(hipStreamSynchronize(ctx.stream));
+  return NTLP_OK;
 }
 
 int ntlp_gpu_particles_get_records(void* records, int64_t n) {
   CHK(need_init());
   if (n != ctx.n || (n > 0 && !records)) return fail(NTLP_E_INVALID, "bad record buffer");
-  std::vector<double> soa((size_t)n * NTLP_NREAL);
-  std::vector<int64_t> mult((size_t)n);
-  std::vector<int32_t> pidx((size_t)n), procidx((size_t)n);
-  CHK(ntlp_gpu_particles_get(soa.data(), mult.data(), pidx.data(), procidx.data(), n));
-  unsigned char* base = (unsigned char*)records;
-  for (int64_t i = 0; i < n; ++i) {
-    unsigned char* r = base + i * NTLP_RECORD_BYTES;
-    const int32_t ints[4] = {pidx[i], procidx[i], -1, -1};
-    double reals[kRecReals];
-    for (int k = 0; k < kRecReals; ++k) reals[k] = kRecCol[k] >= 0 ? soa[(size_t)kRecCol[k] * n + i] : 0.0;
-    memcpy(r, ints, 16);
-    memcpy(r + 16, reals, 8 * kRecReals);
-    memcpy(r + 16 + 8 * kRecReals, &mult[i], 8);
-    memset(r + 16 + 8 * kRecReals + 8, 0, 16);
+  if (ctx.state_bad)
+    return fail(NTLP_E_STATE, "a failed step call left the droplets inconsistent: put them again");
+  CHK(flush_diag());
+  if (n == 0) return NTLP_OK;
+  CHK(xfer_stage(kRecWords, kRecWords * n));
+  const int64_t per = std::min(n, ctx.xfer_cap / kRecWords);
+  const ColumnPlace pl = record_places();
+  const int32_t* slot = nullptr;
+  if (!ctx.home_identity) {  // put index -> slot
+    int32_t* inv = (int32_t*)ctx.col_tmp;
+    CHK(launch("get", [&] { k_invert<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, ctx.stream>>>(ctx.home[ctx.cur], n, inv); }));
+    slot = inv;
   }
+  unsigned char* base = (unsigned char*)records;
+  for (int64_t i = 0; i < n; i += per) {
+    const int64_t m = std::min(per, n - i);
+    CHK(launch("get", [&] {
+      k_records_out<<<(unsigned)((m + kRecTile - 1) / kRecTile), kBlock, 0, ctx.stream>>>(
+          (uint64_t*)ctx.xfer, i, m, pl, ctx.cap, ctx.hot[ctx.cur], ctx.cold, ctx.mult[ctx.cur], ctx.pidx, ctx.procidx, slot);
+    }));
+    HIPCHK(hipMemcpyAsync(base + i * NTLP_RECORD_BYTES, ctx.xfer, (size_t)m * NTLP_RECORD_BYTES, hipMemcpyDeviceToHost,
+                          ctx.stream));
+  }
+  HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
 
@@ -1553,9 +1591,8 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
     return fail(NTLP_E_INVALID, "apply_particle_coupling takes x-pencil or core arrays");
   const int nx = ctx.g.nnx, ny = ctx.g.nny, nz = ctx.g.nnz;
   const int64_t elems = layout == NTLP_LAYOUT_XPENCIL ? (int64_t)(nx + 2) * ny * (nz + 2) : (int64_t)(nz + 2) * ny * nx;
-  double* stage[2] = {nullptr, nullptr};
-  int rc = dalloc(stage[0], elems, "field staging");
-  if (!rc) rc = dalloc(stage[1], elems, "field staging");
+  int rc = xfer_stage(2 * elems, 2 * elems);
+  double* stage[2] = {ctx.xfer, ctx.xfer + elems};
   double* host[2] = {T, q};
   for (int i = 0; i < 2 && !rc; ++i)
     if (hipMemcpyAsync(stage[i], host[i], sizeof(double) * elems, hipMemcpyHostToDevice, ctx.stream) != hipSuccess)
@@ -1575,13 +1612,11 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
     const double* stg = stage[i];
     if (!rc)
       rc = launch("fill_ext", [&] {
-        if (layout == NTLP_LAYOUT_CORE) k_fill_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, nx, ny, nz);
-        else k_xpencil_to_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, nx, ny, nz);
+        if (layout == NTLP_LAYOUT_CORE) k_fill_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, nullptr, nx, ny, nz);
+        else k_xpencil_to_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, nullptr, nx, ny, nz);
       });
   }
   if (hipStreamSynchronize(ctx.stream) != hipSuccess && !rc) rc = fail(NTLP_E_HIP, "apply_particle_coupling failed");
-  dfree(stage[0]);
-  dfree(stage[1]);
   return rc;
 }
 
