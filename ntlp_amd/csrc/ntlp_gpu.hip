@@ -10,10 +10,13 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
 #include "../../include/ntlp_gpu.h"
+#include "host_copy.hpp"
 #include "kernels.hpp"
 
 using namespace ntlp;
@@ -59,6 +62,8 @@ struct Ctx {
   float* f32[3] = {};
   double* xfer = nullptr;  // staging of host transfers (see xfer_stage)
   int64_t xfer_cap = 0;    // its doubles
+  std::unique_ptr<HostLink> link;  // pinned slots of large host copies
+  bool no_link = false;            // they could not be had
   bool have_fields = false;
   int64_t ext_elems = 0;
   // droplets
@@ -271,6 +276,43 @@ int fill_i32(int32_t* p, int64_t n, int32_t v) {
   return launch("fill", [&] { k_fill_i32<<<grid_flat(n), kBlock, 0, ctx.stream>>>(p, n, v); });
 }
 
+// Whether a copy of host memory goes through the pinned slots: large ones of
+// pageable memory.
+bool use_link(const void* host, size_t bytes) {
+  if (bytes < HostLink::kDirect || ctx.no_link) return false;
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, host) == hipSuccess) {
+    if (at.type != hipMemoryTypeUnregistered) return false;  // pinned: the link reads or writes it itself
+  } else {
+    (void)hipGetLastError();  // how older runtimes say that they do not know the address
+  }
+  if (!ctx.link) {
+    std::unique_ptr<HostLink> l(new (std::nothrow) HostLink());
+    if (!l || l->open() != hipSuccess) {
+      (void)hipGetLastError();
+      if (l) l->close();
+      ctx.no_link = true;
+      return false;
+    }
+    ctx.link = std::move(l);
+  }
+  return true;
+}
+
+// Copies on the library stream.  to_device: src may be reused on return unless
+// it is pinned (the caller synchronises before it hands it back).  to_host:
+// dst is complete after the next synchronisation.
+int to_device(void* dst, const void* src, size_t bytes) {
+  if (use_link(src, bytes)) HIPCHK(ctx.link->up(dst, src, bytes, ctx.stream));
+  else HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx.stream));
+  return 0;
+}
+int to_host(void* dst, const void* src, size_t bytes) {
+  if (use_link(dst, bytes)) HIPCHK(ctx.link->down(dst, src, bytes, ctx.stream));
+  else HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx.stream));
+  return 0;
+}
+
 // The staging buffer with room for at least `least` doubles, `want` if that
 // stays below kXferBytes.  It is kept until the context is released: allocated
 // and freed on each call it cost 40 to 260 us.  Its users leave it to the next
@@ -321,6 +363,7 @@ void release_all() {
   }
   ctx.pending.clear();
   ctx.totals.clear();
+  if (ctx.link) ctx.link->close();
   if (ctx.stream) (void)hipStreamDestroy(ctx.stream);
   ctx = Ctx();
 }
@@ -1065,11 +1108,11 @@ int ntlp_gpu_set_fields(const double* u, const double* v, const double* w, const
     double* dst = ctx.ext[f];
     float* o = f < 3 ? ctx.f32[f] : nullptr;
     if (layout == NTLP_LAYOUT_EXT) {
-      HIPCHK(hipMemcpyAsync(dst, in[f], sizeof(double) * in_elems, hipMemcpyHostToDevice, ctx.stream));
+      CHK(to_device(dst, in[f], sizeof(double) * in_elems));
       if (o) CHK(launch("to_f32", [&] { k_to_f32<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(dst, o, ctx.ext_elems); }));
       continue;
     }
-    HIPCHK(hipMemcpyAsync(ctx.xfer, in[f], sizeof(double) * in_elems, hipMemcpyHostToDevice, ctx.stream));
+    CHK(to_device(ctx.xfer, in[f], sizeof(double) * in_elems));
     const double* stg = ctx.xfer;
     CHK(launch("fill_ext", [&] {
       if (layout == NTLP_LAYOUT_CORE) k_fill_ext<<<grid_flat(ctx.ext_elems), kBlock, 0, ctx.stream>>>(stg, dst, o, nx, ny, nz);
@@ -1174,16 +1217,16 @@ int ntlp_gpu_particles_put(const double* soa, const int64_t* mult, const int32_t
   const ColumnPlace pl = column_places();
   for (int c = 0; c < NTLP_NREAL; c += per) {
     const int nc = std::min(per, NTLP_NREAL - c);
-    HIPCHK(hipMemcpyAsync(ctx.xfer, soa + (int64_t)c * n, sizeof(double) * nc * n, hipMemcpyHostToDevice, ctx.stream));
+    CHK(to_device(ctx.xfer, soa + (int64_t)c * n, sizeof(double) * nc * n));
     CHK(launch("put", [&] {
       k_columns_in<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(ctx.xfer, c, pl, n, ctx.cap,
                                                                                               ctx.hot[0], ctx.cold);
     }));
   }
-  HIPCHK(hipMemcpyAsync(ctx.mult[0], mult, sizeof(int64_t) * n, hipMemcpyHostToDevice, ctx.stream));
-  if (pidx) HIPCHK(hipMemcpyAsync(ctx.pidx, pidx, sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx.stream));
+  CHK(to_device(ctx.mult[0], mult, sizeof(int64_t) * n));
+  if (pidx) CHK(to_device(ctx.pidx, pidx, sizeof(int32_t) * n));
   else CHK(fill_i32(ctx.pidx, n, 0));
-  if (procidx) HIPCHK(hipMemcpyAsync(ctx.procidx, procidx, sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx.stream));
+  if (procidx) CHK(to_device(ctx.procidx, procidx, sizeof(int32_t) * n));
   else CHK(fill_i32(ctx.procidx, n, 0));
   CHK(launch("iota", [&] { k_iota<<<grid_flat(n), kBlock, 0, ctx.stream>>>(ctx.home[0], n); }));
   HIPCHK(hipStreamSynchronize(ctx.stream));
@@ -1209,7 +1252,7 @@ int ntlp_gpu_particles_get(double* soa, int64_t* mult, int32_t* pidx, int32_t* p
         k_columns_out<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(
             ctx.xfer, c, pl, n, ctx.cap, ctx.hot[ctx.cur], ctx.cold, hm);
       }));
-      HIPCHK(hipMemcpyAsync(soa + (int64_t)c * n, ctx.xfer, sizeof(double) * nc * n, hipMemcpyDeviceToHost, ctx.stream));
+      CHK(to_host(soa + (int64_t)c * n, ctx.xfer, sizeof(double) * nc * n));
     }
   }
   if (mult) {
@@ -1219,10 +1262,10 @@ int ntlp_gpu_particles_get(double* soa, int64_t* mult, int32_t* pidx, int32_t* p
       CHK(launch("get", [&] { k_scatter_col_i64<<<grid_flat(n), kBlock, 0, ctx.stream>>>(col, home, n, tmp); }));
       col = tmp;
     }
-    HIPCHK(hipMemcpyAsync(mult, col, sizeof(int64_t) * n, hipMemcpyDeviceToHost, ctx.stream));
+    CHK(to_host(mult, col, sizeof(int64_t) * n));
   }
-  if (pidx) HIPCHK(hipMemcpyAsync(pidx, ctx.pidx, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx.stream));
-  if (procidx) HIPCHK(hipMemcpyAsync(procidx, ctx.procidx, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx.stream));
+  if (pidx) CHK(to_host(pidx, ctx.pidx, sizeof(int32_t) * n));
+  if (procidx) CHK(to_host(procidx, ctx.procidx, sizeof(int32_t) * n));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
@@ -1265,8 +1308,7 @@ int ntlp_gpu_particles_put_records(const void* records, int64_t n) {
   const unsigned char* base = (const unsigned char*)records;
   for (int64_t i = 0; i < n; i += per) {
     const int64_t m = std::min(per, n - i);
-    HIPCHK(hipMemcpyAsync(ctx.xfer, base + i * NTLP_RECORD_BYTES, (size_t)m * NTLP_RECORD_BYTES, hipMemcpyHostToDevice,
-                          ctx.stream));
+    CHK(to_device(ctx.xfer, base + i * NTLP_RECORD_BYTES, (size_t)m * NTLP_RECORD_BYTES));
     CHK(launch("put", [&] {
       k_records_in<<<(unsigned)((m + kRecTile - 1) / kRecTile), kBlock, 0, ctx.stream>>>(
           (const uint64_t*)ctx.xfer, i, m, pl, ctx.cap, ctx.hot[0], ctx.cold, ctx.mult[0], ctx.pidx, ctx.procidx);
@@ -1300,8 +1342,7 @@ int ntlp_gpu_particles_get_records(void* records, int64_t n) {
       k_records_out<<<(unsigned)((m + kRecTile - 1) / kRecTile), kBlock, 0, ctx.stream>>>(
           (uint64_t*)ctx.xfer, i, m, pl, ctx.cap, ctx.hot[ctx.cur], ctx.cold, ctx.mult[ctx.cur], ctx.pidx, ctx.procidx, slot);
     }));
-    HIPCHK(hipMemcpyAsync(base + i * NTLP_RECORD_BYTES, ctx.xfer, (size_t)m * NTLP_RECORD_BYTES, hipMemcpyDeviceToHost,
-                          ctx.stream));
+    CHK(to_host(base + i * NTLP_RECORD_BYTES, ctx.xfer, (size_t)m * NTLP_RECORD_BYTES));
   }
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
@@ -1389,10 +1430,8 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
   int64_t* d_start = nullptr;
   CHK(dalloc(d_ens, nens, "ensembles"));
   int rc = dalloc(d_start, nens + 1, "ensemble starts");
-  if (!rc && (hipMemcpyAsync(d_ens, de.data(), sizeof(DevEnsemble) * nens, hipMemcpyHostToDevice, ctx.stream) !=
-                  hipSuccess ||
-              hipMemcpyAsync(d_start, start.data(), sizeof(int64_t) * (nens + 1), hipMemcpyHostToDevice, ctx.stream) !=
-                  hipSuccess))
+  if (!rc && (to_device(d_ens, de.data(), sizeof(DevEnsemble) * nens) != 0 ||
+              to_device(d_start, start.data(), sizeof(int64_t) * (nens + 1)) != 0))
     rc = fail(NTLP_E_HIP, "ensemble upload failed");
   GenArgs a;
   a.g = ctx.g;
@@ -1450,11 +1489,10 @@ int ntlp_gpu_particles_get_column(int32_t column, double* out, int64_t n) {
     double* tmp = ctx.col_tmp;
     const int32_t* hm = ctx.home_identity ? nullptr : ctx.home[ctx.cur];
     CHK(launch("get", [&] { k_unpack_hot<<<grid_flat(n), kBlock, 0, ctx.stream>>>(hot, hc, hm, n, tmp); }));
-    HIPCHK(hipMemcpyAsync(out, tmp, sizeof(double) * n, hipMemcpyDeviceToHost, ctx.stream));
+    CHK(to_host(out, tmp, sizeof(double) * n));
   } else {
     CHK(flush_diag());
-    HIPCHK(hipMemcpyAsync(out, ctx.cold + (int64_t)cold_of(column) * ctx.cap, sizeof(double) * n,
-                          hipMemcpyDeviceToHost, ctx.stream));
+    CHK(to_host(out, ctx.cold + (int64_t)cold_of(column) * ctx.cap, sizeof(double) * n));
   }
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
@@ -1539,7 +1577,7 @@ int ntlp_gpu_particle_coupling_update(double* src_out, int32_t deterministic) {
     ctx.src_valid = true;
     ctx.xsrc_valid = false;
     if (src_out)
-      HIPCHK(hipMemcpyAsync(src_out, ctx.src, sizeof(double) * 6 * ctx.nsrc, hipMemcpyDeviceToHost, ctx.stream));
+      CHK(to_host(src_out, ctx.src, sizeof(double) * 6 * ctx.nsrc));
     HIPCHK(hipStreamSynchronize(ctx.stream));
     return NTLP_OK;
   }
@@ -1555,7 +1593,7 @@ int ntlp_gpu_particle_coupling_update(double* src_out, int32_t deterministic) {
   else if (deterministic == 2) CHK(scatter_atomic());
   else CHK(scatter_tile());
   if (src_out)
-    HIPCHK(hipMemcpyAsync(src_out, ctx.src, sizeof(double) * 6 * ctx.nsrc, hipMemcpyDeviceToHost, ctx.stream));
+    CHK(to_host(src_out, ctx.src, sizeof(double) * 6 * ctx.nsrc));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
@@ -1575,8 +1613,7 @@ int ntlp_gpu_particle_coupling_exchange(double* partsrc, double* partTsrc, doubl
   const int first[4] = {0, 3, 4, 5}, count[4] = {3, 1, 1, 1};
   for (int i = 0; i < 4; ++i)
     if (outs[i])
-      HIPCHK(hipMemcpyAsync(outs[i], ctx.xsrc + first[i] * nf, sizeof(double) * count[i] * nf, hipMemcpyDeviceToHost,
-                            ctx.stream));
+      CHK(to_host(outs[i], ctx.xsrc + first[i] * nf, sizeof(double) * count[i] * nf));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   ctx.xsrc_valid = true;
   return NTLP_OK;
@@ -1595,7 +1632,7 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
   double* stage[2] = {ctx.xfer, ctx.xfer + elems};
   double* host[2] = {T, q};
   for (int i = 0; i < 2 && !rc; ++i)
-    if (hipMemcpyAsync(stage[i], host[i], sizeof(double) * elems, hipMemcpyHostToDevice, ctx.stream) != hipSuccess)
+    if (to_device(stage[i], host[i], sizeof(double) * elems) != 0)
       rc = fail(NTLP_E_HIP, "upload of T/q failed");
   if (!rc) {
     const int xp = layout == NTLP_LAYOUT_XPENCIL;
@@ -1605,7 +1642,7 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
     });
   }
   for (int i = 0; i < 2 && !rc; ++i) {
-    if (hipMemcpyAsync(host[i], stage[i], sizeof(double) * elems, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess)
+    if (to_host(host[i], stage[i], sizeof(double) * elems) != 0)
       rc = fail(NTLP_E_HIP, "download of T/q failed");
     // the resident T (ext 3) and q (ext 4) the next step gathers
     double* dst = ctx.ext[3 + i];
@@ -1623,7 +1660,7 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
 int ntlp_gpu_get_sources(double* src_out) {
   CHK(need_init());
   if (!src_out) return fail(NTLP_E_INVALID, "null output");
-  HIPCHK(hipMemcpyAsync(src_out, ctx.src, sizeof(double) * 6 * ctx.nsrc, hipMemcpyDeviceToHost, ctx.stream));
+  CHK(to_host(src_out, ctx.src, sizeof(double) * 6 * ctx.nsrc));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
@@ -1646,15 +1683,15 @@ int ntlp_gpu_bin(int32_t* cellidx, int32_t* counts, int32_t* offsets, int32_t* p
   if (rc == 0 && cellidx) {
     const int32_t* home = ctx.home[ctx.cur];
     rc = launch("bin_out", [&] { k_scatter_home_i32x4<<<grid_flat(n), kBlock, 0, ctx.stream>>>(ci_dev, home, n, ci_put); });
-    if (rc == 0 && hipMemcpyAsync(cellidx, ci_put, sizeof(int32_t) * 4 * n, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess)
+    if (rc == 0 && to_host(cellidx, ci_put, sizeof(int32_t) * 4 * n) != 0)
       rc = fail(NTLP_E_HIP, "copy of cell indices failed");
   }
   if (rc == 0 && offsets &&
-      hipMemcpyAsync(offsets, ctx.offsets, sizeof(int32_t) * (ctx.ncell + 1), hipMemcpyDeviceToHost, ctx.stream) != hipSuccess)
+      to_host(offsets, ctx.offsets, sizeof(int32_t) * (ctx.ncell + 1)) != 0)
     rc = fail(NTLP_E_HIP, "copy of offsets failed");
   if (rc == 0 && counts) {
     std::vector<int32_t> off((size_t)ctx.ncell + 1);
-    if (hipMemcpyAsync(off.data(), ctx.offsets, sizeof(int32_t) * (ctx.ncell + 1), hipMemcpyDeviceToHost, ctx.stream) != hipSuccess ||
+    if (to_host(off.data(), ctx.offsets, sizeof(int32_t) * (ctx.ncell + 1)) != 0 ||
         hipStreamSynchronize(ctx.stream) != hipSuccess)
       rc = fail(NTLP_E_HIP, "copy of offsets failed");
     else
@@ -1669,7 +1706,7 @@ int ntlp_gpu_bin(int32_t* cellidx, int32_t* counts, int32_t* offsets, int32_t* p
       rc = fail(NTLP_E_HIP, "perm copy failed");
     const int32_t* home = ctx.home[ctx.cur];
     if (rc == 0) rc = launch("bin_out", [&] { k_map_home<<<grid_flat(n), kBlock, 0, ctx.stream>>>(pp, home, n); });
-    if (rc == 0 && hipMemcpyAsync(perm, pp, sizeof(int32_t) * n, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess)
+    if (rc == 0 && to_host(perm, pp, sizeof(int32_t) * n) != 0)
       rc = fail(NTLP_E_HIP, "copy of perm failed");
     if (hipStreamSynchronize(ctx.stream) != hipSuccess && rc == 0) rc = fail(NTLP_E_HIP, "sync failed");
     dfree(pp);
@@ -1698,7 +1735,7 @@ int ntlp_gpu_wcell_counts(int32_t* num_array) {
     b.cellidx = nullptr;
     rc = launch("wcells", [&] { k_wcells<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(b, d); });
   }
-  if (rc == 0 && hipMemcpyAsync(num_array, d, sizeof(int32_t) * nw, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess)
+  if (rc == 0 && to_host(num_array, d, sizeof(int32_t) * nw) != 0)
     rc = fail(NTLP_E_HIP, "copy failed");
   if (hipStreamSynchronize(ctx.stream) != hipSuccess && rc == 0) rc = fail(NTLP_E_HIP, "sync failed");
   dfree(d);
@@ -1724,7 +1761,7 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
   if (!rc && (hipMemsetAsync(rad, 0, sizeof(double) * ncell, ctx.stream) != hipSuccess ||
               hipMemsetAsync(nc, 0, sizeof(double) * ncell, ctx.stream) != hipSuccess ||
               hipMemsetAsync(num, 0, sizeof(int32_t) * ncell, ctx.stream) != hipSuccess ||
-              hipMemcpyAsync(res, &start, sizeof(double), hipMemcpyHostToDevice, ctx.stream) != hipSuccess))
+              to_device(res, &start, sizeof(double)) != 0))
     rc = fail(NTLP_E_HIP, "tauc_min set-up failed");
   if (!rc) {
     BinArgs b;
@@ -1738,7 +1775,7 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
   if (!rc)
     rc = launch("tauc", [&] { k_tauc_min<<<grid_flat(ncell), kBlock, 0, ctx.stream>>>(ctx.g, ctx.C, rad, num, nc, res); });
   double m = 0.0;
-  if (!rc && (hipMemcpyAsync(&m, res, sizeof(double), hipMemcpyDeviceToHost, ctx.stream) != hipSuccess ||
+  if (!rc && (to_host(&m, res, sizeof(double)) != 0 ||
               hipStreamSynchronize(ctx.stream) != hipSuccess))
     rc = fail(NTLP_E_HIP, "tauc_min failed");
   dfree(rad);
@@ -1762,10 +1799,9 @@ int ntlp_gpu_particle_xy_stats(double* s0, double* s1, double* lwp) {
   if (!rc) rc = dalloc(out1, 24 * sh.nz2, "statistics");
   if (!rc) rc = dalloc(lw, (int64_t)ctx.g.nnx * ctx.g.nny, "LWP");
   if (!rc) rc = stats_launch(sh, cold, part0, part1, out0, out1, lw, true);
-  if (!rc && ((s0 && hipMemcpyAsync(s0, out0, sizeof(double) * kStats0, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess) ||
-              (s1 && hipMemcpyAsync(s1, out1, sizeof(double) * 24 * sh.nz2, hipMemcpyDeviceToHost, ctx.stream) != hipSuccess) ||
-              (lwp && hipMemcpyAsync(lwp, lw, sizeof(double) * ctx.g.nnx * ctx.g.nny, hipMemcpyDeviceToHost,
-                                     ctx.stream) != hipSuccess) ||
+  if (!rc && ((s0 && to_host(s0, out0, sizeof(double) * kStats0) != 0) ||
+              (s1 && to_host(s1, out1, sizeof(double) * 24 * sh.nz2) != 0) ||
+              (lwp && to_host(lwp, lw, sizeof(double) * ctx.g.nnx * ctx.g.nny) != 0) ||
               hipStreamSynchronize(ctx.stream) != hipSuccess))
     rc = fail(NTLP_E_HIP, "statistics copy failed");
   dfree(part0);
@@ -1813,7 +1849,7 @@ int ntlp_gpu_step(int32_t mode, int32_t prec, int32_t nsteps, int32_t it0) {
 int ntlp_gpu_counters(ntlp_counters* out, int32_t reset) {
   CHK(need_init());
   unsigned long long row[kTallyWidth];
-  HIPCHK(hipMemcpyAsync(row, ctx.tally_totals, sizeof(row), hipMemcpyDeviceToHost, ctx.stream));
+  CHK(to_host(row, ctx.tally_totals, sizeof(row)));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   if (out) {
     memset(out, 0, sizeof(*out));
@@ -1845,7 +1881,7 @@ int ntlp_gpu_be_flux(double* pflux, double* pmassflux, double* penegflux) {
   double* outs[3] = {pflux, pmassflux, penegflux};
   for (int k = 0; k < 3; ++k)
     if (outs[k])
-      HIPCHK(hipMemcpyAsync(outs[k], f + (int64_t)k * nlev, sizeof(double) * nlev, hipMemcpyDeviceToHost, ctx.stream));
+      CHK(to_host(outs[k], f + (int64_t)k * nlev, sizeof(double) * nlev));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
 }
@@ -1855,7 +1891,7 @@ int ntlp_gpu_step_counters(int64_t* rows_out, int32_t max_rows) {
   if (!rows_out || max_rows <= 0) return fail(NTLP_E_INVALID, "bad output");
   const int64_t nr = std::min<int64_t>(std::min<int64_t>(ctx.step_row, kTallyRows - 1), max_rows);
   std::vector<unsigned long long> rows((size_t)kTallyRows * kTallyWidth);
-  HIPCHK(hipMemcpyAsync(rows.data(), ctx.tally, sizeof(unsigned long long) * rows.size(), hipMemcpyDeviceToHost, ctx.stream));
+  CHK(to_host(rows.data(), ctx.tally, sizeof(unsigned long long) * rows.size()));
   HIPCHK(hipStreamSynchronize(ctx.stream));
   // rows 1..step_row hold the steps in order (row 0 is the pre-step row)
   for (int64_t r = 0; r < nr; ++r) {

@@ -65,3 +65,37 @@ def test_round_trips(ctx, n):
     assert np.array_equal(r[:, :2].copy().view(np.int32)[:, 0], p.pidx)
     for c in ("x", "Tp", "ufz"):
         assert np.array_equal(s.column(c), q[c])
+
+
+@pytest.mark.parametrize("mb", [0.9, 1.0, 1.1, 2.0, 3.99, 4.0, 16.0, 16.01, 33.3])
+def test_large_fields_and_sources_pageable(mb):
+    """Copies below, at and above the sizes at which they go through the pinned slots (1 MB) and wrap round them
+    (4 x 4 MB): fields in by both layouts and sources out give the same bits."""
+    nz = 30
+    nx = 16
+    ny = max(2, int(round(mb * 1e6 / 8 / ((nz + 2) * nx))))
+    g = Grid.uniform(nx, ny, nz, 0.02, 0.02, 0.02)
+    rng = np.random.default_rng(ny)
+    f = [rng.standard_normal((nx, ny, nz + 2)) for _ in range(3)] + [300 + rng.random((nx, ny, nz + 2)), 0.02 * rng.random((nx, ny, nz + 2))]
+    n = int(mb * 1e6 / 8)
+    out = []
+    for xp in (False, True):
+        s = DropletStep(g, Consts(dt=1e-6), Flags())
+        if xp:
+            x = [np.zeros((nz + 2, ny, nx + 2)) for _ in f]
+            for a, b in zip(x, f):
+                a[:, :, :nx] = b.transpose(2, 1, 0)
+            s.set_fields(*x, layout=2)
+        else:
+            s.set_fields(*f)
+        s.put(droplets(s, n))
+        s.interp(set_vp=True, set_tp=True)
+        s.step(MODE_RK3, PREC_FP64, nsteps=1, it0=2)
+        src = s.sources()
+        ex = s.particle_coupling_exchange()
+        out.append((s.get().soa, src, ex))
+        s.close()
+    (a, sa, ea), (b, sb, eb) = out
+    assert np.array_equal(a, b)
+    for u, v in zip((sa, *ea), (sb, *eb)):  # sums in an order that varies
+        assert np.all(np.isfinite(u)) and np.max(np.abs(u - v)) <= 1e-12 * np.max(np.abs(u))
