@@ -1212,7 +1212,64 @@ __global__ void __launch_bounds__(kBlock) k_keys(BinArgs a) {
   count_key(a.counts, key, valid);
 }
 
-// calc_tauc_min's num_array over w cells (particles.f90:3320-3339).
+// calc_tauc_min's num_array over w cells (particles.f90:3320-3339).  On grids
+// whose levels interleave, the droplets of w cell (i, j, kc) lie in the u cells
+// (i, j, kc-1) and (i, j, kc), consecutive keys, so their sort (offsets + perm)
+// holds them in one run of slots: every w cell looks through its run, without
+// atomics or a cleared array.  Slots of a first or last column (keys clamped
+// into the box) are checked for their own column as well.
+struct WcellArgs {
+  DevGrid g;
+  const double* hot;
+  const int64_t* mult;
+  const int32_t* perm;     // sorted index -> slot
+  const int32_t* offsets;  // u-cell offsets of the sort
+};
+
+// f(slot) for every droplet of the w cell (i, j, kc): 0-based i and j, 1-based kc
+template <class F>
+__device__ __forceinline__ void each_of_wcell(const WcellArgs& a, const double* s_z, int i, int j, int kc, F f) {
+  const int key = kc - 1 + (a.g.nnz + 1) * (j + (a.g.nny + 1) * i);
+  const int b = a.offsets[key], e = a.offsets[key + 2];
+  const double lo = s_z[kc - 1], hi = s_z[kc];
+  const bool edge = i == 0 || j == 0;
+  for (int p = b; p < e; ++p) {
+    const int64_t t = a.perm[p];
+    const double z = a.hot[hix(kHZ, t)];
+    if (!(hi > z) || lo > z) continue;  // first_gt(z) is another level
+    if (edge && ((int)floor(a.hot[hix(kHX, t)] / a.g.dx) != i || (int)floor(a.hot[hix(kHY, t)] / a.g.dy) != j)) continue;
+    f(t);
+  }
+}
+
+// Bound by the latency of the run's loads (offsets, perm, z): a workgroup takes
+// kWcellI x kWcellK cells of one (j) row, levels along the lanes, where the
+// offsets and the runs are consecutive, and turns them in LDS so that the
+// counts leave in 128-byte pieces along i.  3M droplets on 128^3: 121 us
+// with an atomic for each droplet, 62 us so.
+constexpr int kWcellI = 32, kWcellK = 64;
+__global__ void __launch_bounds__(kBlock) k_wcells_sorted(WcellArgs a, int32_t* num) {
+  __shared__ double s_z[kMaxLevels];
+  __shared__ int32_t s_num[kWcellI][kWcellK + 1];
+  for (int k = threadIdx.x; k < a.g.nnz + 2; k += blockDim.x) s_z[k] = a.g.z[k];
+  __syncthreads();
+  const int nti = (a.g.nnx + kWcellI - 1) / kWcellI, ntk = (a.g.nnz + kWcellK - 1) / kWcellK;
+  const int i0 = (int)(blockIdx.x % nti) * kWcellI, k0 = (int)(blockIdx.x / nti % ntk) * kWcellK;
+  const int j = (int)(blockIdx.x / nti / ntk);
+  const int kk = threadIdx.x % kWcellK;
+  for (int ii = threadIdx.x / kWcellK; ii < kWcellI; ii += kBlock / kWcellK) {
+    int c = 0;
+    if (i0 + ii < a.g.nnx && k0 + kk < a.g.nnz) each_of_wcell(a, s_z, i0 + ii, j, k0 + kk + 1, [&](int64_t) { ++c; });
+    s_num[ii][kk] = c;
+  }
+  __syncthreads();
+  const int io = threadIdx.x % kWcellI;
+  for (int ko = threadIdx.x / kWcellI; ko < kWcellK; ko += kBlock / kWcellI)
+    if (i0 + io < a.g.nnx && k0 + ko < a.g.nnz)
+      num[(i0 + io) + (int64_t)a.g.nnx * (j + (int64_t)a.g.nny * (k0 + ko))] = s_num[io][ko];
+}
+
+// The same for any grid: an atomic for each droplet.
 __global__ void __launch_bounds__(kBlock) k_wcells(BinArgs a, int32_t* num) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   stage_grid(a.g, s_z, s_zz);
@@ -1228,7 +1285,7 @@ __global__ void __launch_bounds__(kBlock) k_wcells(BinArgs a, int32_t* num) {
 
 // ------------------------------------------------------------ statistics
 
-// calc_tauc_min (particles.f90:3310-3368), first half: radius sum, count and
+// calc_tauc_min (particles.f90:3310-3368), over any grid, first half: radius sum, count and
 // multiplicity sum per w cell (ipt, jpt, kc); droplets outside (1:nnx,
 // 1:nny, 1:nnz) are not counted.
 __global__ void __launch_bounds__(kBlock) k_tauc_accum(BinArgs a, const int64_t* mult, double* rad, int32_t* num,
@@ -1248,30 +1305,61 @@ __global__ void __launch_bounds__(kBlock) k_tauc_accum(BinArgs a, const int64_t*
   atomicAdd(&nc[e], (double)mult[t]);
 }
 
-// Second half: the smallest 1/(denom + 1e-10) over occupied cells, as the
-// bit pattern of a positive double (ordered like the value) in *out.
-__global__ void __launch_bounds__(kBlock) k_tauc_min(DevGrid g, DevConsts C, const double* rad, const int32_t* num,
-                                                     const double* nc, unsigned long long* out) {
+// The smallest 1/(denom + 1e-10) over occupied cells, as the bit pattern of a
+// positive double (ordered like the value) in *out.
+__device__ __forceinline__ double tauc_of(const DevGrid& g, const DevConsts& C, int iz, double rad, int32_t num, double nc) {
+  const double radavg = rad / (double)num;
+  const double Nc = nc / (g.dx * g.dy * g.dzw[iz]);
+  const double denom = C.pi2 * (C.nuf / C.Sc) * 2.0 * radavg * Nc;
+  return 1.0 / (denom + 1.0e-10);
+}
+
+__device__ __forceinline__ void tauc_close(double m, unsigned long long* out) {
   __shared__ double s_min[kBlock / 64];
-  const int64_t ncell = (int64_t)g.nnx * g.nny * g.nnz;
-  double m = 1.0e10;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ncell; e += (int64_t)gridDim.x * blockDim.x) {
-    if (num[e] != 0) {
-      const int iz = (int)(e / ((int64_t)g.nnx * g.nny)) + 1;
-      const double radavg = rad[e] / (double)num[e];
-      const double Nc = nc[e] / (g.dx * g.dy * g.dzw[iz]);
-      const double denom = C.pi2 * (C.nuf / C.Sc) * 2.0 * radavg * Nc;
-      m = fmin(m, 1.0 / (denom + 1.0e-10));
-    }
-  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
   if (lane_id() == 0) s_min[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < (int)(blockDim.x >> 6); ++w) m = fmin(m, s_min[w]);
-    atomicMin(out, (unsigned long long)__double_as_longlong(m));
+    // most workgroups find a smaller value there already
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    if (bits < __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(out, bits);
   }
+}
+
+__global__ void __launch_bounds__(kBlock) k_tauc_min(DevGrid g, DevConsts C, const double* rad, const int32_t* num,
+                                                     const double* nc, unsigned long long* out) {
+  const int64_t ncell = (int64_t)g.nnx * g.nny * g.nnz;
+  double m = 1.0e10;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ncell; e += (int64_t)gridDim.x * blockDim.x)
+    if (num[e] != 0) m = fmin(m, tauc_of(g, C, (int)(e / ((int64_t)g.nnx * g.nny)) + 1, rad[e], num[e], nc[e]));
+  tauc_close(m, out);
+}
+
+// Both halves at once where a w cell's droplets are one run of the sort: no
+// cell arrays to clear, to add to and to read back.  Levels along the lanes;
+// bound by the latency of the run's loads.  3M droplets on 128^3: 480 us
+// with three atomics for each droplet, 63 us so.
+__global__ void __launch_bounds__(kBlock) k_tauc_sorted(WcellArgs a, DevConsts C, unsigned long long* out) {
+  __shared__ double s_z[kMaxLevels];
+  for (int k = threadIdx.x; k < a.g.nnz + 2; k += blockDim.x) s_z[k] = a.g.z[k];
+  __syncthreads();
+  const int64_t ncell = (int64_t)a.g.nnx * a.g.nny * a.g.nnz;
+  double m = 1.0e10;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ncell; e += (int64_t)gridDim.x * blockDim.x) {
+    const int kc = (int)(e % a.g.nnz) + 1;
+    const int col = (int)(e / a.g.nnz);
+    double rad = 0.0, nc = 0.0;
+    int32_t num = 0;
+    each_of_wcell(a, s_z, col / a.g.nny, col % a.g.nny, kc, [&](int64_t t) {
+      rad += a.hot[hix(kHR, t)];
+      nc += (double)a.mult[t];
+      ++num;
+    });
+    if (num != 0) m = fmin(m, tauc_of(a.g, C, kc, rad, num, nc));
+  }
+  tauc_close(m, out);
 }
 
 // particle_xy_stats (particles.f90:3370-3770): the droplet loops.  Each of
@@ -1280,8 +1368,16 @@ __global__ void __launch_bounds__(kBlock) k_tauc_min(DevGrid g, DevConsts C, con
 //    minima, starting from the reference's initial values), reduced in LDS;
 //  - quantities q0..q0+nq-1 of the 24 per-level sums of statsvec1 in LDS;
 // and writes them to its row of `part`; LWP(ipt, jpt) is added with global
-// atomics.  k_xy_reduce then sums the rows in a fixed order.
+// atomics, one a wave and column for the first two columns that the wave meets
+// (in sorted slots a wave stays in one or two, and 64 additions to one word
+// are served one after the other) and one a droplet beyond.  k_xy_reduce then
+// sums the rows in a fixed order.
+// Bound by the LDS atomics and the latency of the loads: the rows stay few (each
+// is read back), so a workgroup has up to kStatsBlock threads, four waves for
+// each SIMD of its compute unit.  3M droplets on 128^3: 430 us with 256
+// threads and an LWP atomic for each droplet, 126 us so.
 constexpr int kStats0 = 21;
+constexpr int kStatsBlock = 1024;
 struct StatsArgs {
   DevGrid g;
   DevConsts C;
@@ -1295,10 +1391,10 @@ struct StatsArgs {
   double* lwp;       // [nny][nnx] (pass 0 only)
 };
 
-__global__ void __launch_bounds__(kBlock) k_xy_stats(StatsArgs a) {
+__global__ void __launch_bounds__(kStatsBlock) k_xy_stats(StatsArgs a) {
   extern __shared__ double s_lvl[];  // [nq][nnz+2]
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
-  __shared__ double s_red[kBlock / 64][kStats0];
+  __shared__ double s_red[kStatsBlock / 64][kStats0];
   stage_grid(a.g, s_z, s_zz);
   const int nz2 = a.g.nnz + 2;
   for (int i = threadIdx.x; i < a.nq * nz2; i += blockDim.x) s_lvl[i] = 0.0;
@@ -1309,46 +1405,65 @@ __global__ void __launch_bounds__(kBlock) k_xy_stats(StatsArgs a) {
   const int64_t chunk = (a.n + gridDim.x - 1) / gridDim.x;
   const int64_t t0 = (int64_t)blockIdx.x * chunk, t1 = min(a.n, t0 + chunk);
   const double pi = 4.0 * atan(1.0);
-  for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-    const Drop d = load_drop(a.hot, t);
-    const int64_t h = a.cold.row(t);
-    const double* cold = a.cold.base;
-    const double uf0 = cold[kCUFX * a.cap + h], uf1 = cold[kCUFY * a.cap + h], uf2 = cold[kCUFZ * a.cap + h];
-    const double Tf = cold[kCTF * a.cap + h], qinf = cold[kCQINF * a.cap + h];
-    const double m = (double)a.mult[t];
-    const double mw = a.C.rhow * 4.0 / 3.0 * pi * pow(d.r, 3);
-    if (first) {
-      v0[0] += 1.0;
-      if (d.r > d.rc) v0[1] += 1.0;
-      else v0[2] += 1.0;
-      const double Volp = a.C.pi2 * 2.0 / 3.0 * pow(d.r, 3);
-      const double rhop = (d.m_s + Volp * a.C.rhow) / Volp;
-      const double d0 = d.vx - uf0, d1 = d.vy - uf1, d2 = d.vz - uf2;
-      v0[3] += 2.0 * d.r * sqrt(d0 * d0 + d1 * d1 + d2 * d2) / a.C.nuf;
-      v0[4] += Volp * a.C.rhow;
-      v0[5] += Volp * rhop;
-      v0[6] += Volp;
-      v0[7] += d.r;
-      v0[8] += d.r * d.r;
-      const double mm[6] = {d.r, d.Tp, qinf, d.vx, d.vy, d.vz};
+  for (int64_t tb = t0; tb < t1; tb += blockDim.x) {
+    const int64_t t = tb + threadIdx.x;
+    int col = -1;  // LWP column
+    double water = 0.0;
+    if (t < t1) {
+      const Drop d = load_drop(a.hot, t);
+      const int64_t h = a.cold.row(t);
+      const double* cold = a.cold.base;
+      const double uf0 = cold[kCUFX * a.cap + h], uf1 = cold[kCUFY * a.cap + h], uf2 = cold[kCUFZ * a.cap + h];
+      const double Tf = cold[kCTF * a.cap + h], qinf = cold[kCQINF * a.cap + h];
+      const double m = (double)a.mult[t];
+      const double mw = a.C.rhow * 4.0 / 3.0 * pi * pow(d.r, 3);
+      if (first) {
+        v0[0] += 1.0;
+        if (d.r > d.rc) v0[1] += 1.0;
+        else v0[2] += 1.0;
+        const double Volp = a.C.pi2 * 2.0 / 3.0 * pow(d.r, 3);
+        const double rhop = (d.m_s + Volp * a.C.rhow) / Volp;
+        const double d0 = d.vx - uf0, d1 = d.vy - uf1, d2 = d.vz - uf2;
+        v0[3] += 2.0 * d.r * sqrt(d0 * d0 + d1 * d1 + d2 * d2) / a.C.nuf;
+        v0[4] += Volp * a.C.rhow;
+        v0[5] += Volp * rhop;
+        v0[6] += Volp;
+        v0[7] += d.r;
+        v0[8] += d.r * d.r;
+        const double mm[6] = {d.r, d.Tp, qinf, d.vx, d.vy, d.vz};
 #pragma unroll
-      for (int k = 0; k < 6; ++k) {
-        v0[9 + k] = fmax(v0[9 + k], mm[k]);
-        v0[15 + k] = fmin(v0[15 + k], mm[k]);
+        for (int k = 0; k < 6; ++k) {
+          v0[9 + k] = fmax(v0[9 + k], mm[k]);
+          v0[15 + k] = fmin(v0[15 + k], mm[k]);
+        }
+      }
+      const Cell c = cell_of(a.g, s_z, s_zz, d.x, d.y, d.z);
+      const int kc = wcell_of(a.g, s_z, d.z);
+      if (kc >= 0) {
+        const double q[24] = {1.0, d.vx, d.vy, d.vz, d.vx * d.vx, d.vy * d.vy, d.vz * d.vz, d.vx * d.vz,
+                              uf0, uf1, uf2, uf0 * uf0, uf1 * uf1, uf2 * uf2, d.Tp, d.Tp * d.Tp, Tf,
+                              d.r, d.r * d.r, qinf, d.Tp * d.vz, m, m * mw, cold[kCQSTAR * a.cap + h]};
+#pragma unroll
+        for (int k = 0; k < 24; ++k)
+          if (k >= a.q0 && k < a.q0 + a.nq) atomicAdd(&s_lvl[(k - a.q0) * nz2 + kc], q[k]);
+      }
+      if (first && c.ipt >= 1 && c.ipt <= a.g.nnx && c.jpt >= 1 && c.jpt <= a.g.nny) {
+        col = (c.ipt - 1) + a.g.nnx * (c.jpt - 1);
+        water = m * mw;
       }
     }
-    const Cell c = cell_of(a.g, s_z, s_zz, d.x, d.y, d.z);
-    const int kc = wcell_of(a.g, s_z, d.z);
-    if (kc >= 0) {
-      const double q[24] = {1.0, d.vx, d.vy, d.vz, d.vx * d.vx, d.vy * d.vy, d.vz * d.vz, d.vx * d.vz,
-                            uf0, uf1, uf2, uf0 * uf0, uf1 * uf1, uf2 * uf2, d.Tp, d.Tp * d.Tp, Tf,
-                            d.r, d.r * d.r, qinf, d.Tp * d.vz, m, m * mw, cold[kCQSTAR * a.cap + h]};
+    unsigned long long todo = __ballot(col >= 0);
+    for (int r = 0; r < 2 && todo; ++r) {
+      const int lead = __ffsll((long long)todo) - 1;
+      const bool mine = col == __shfl(col, lead, 64);
+      double v = mine ? water : 0.0;
 #pragma unroll
-      for (int k = 0; k < 24; ++k)
-        if (k >= a.q0 && k < a.q0 + a.nq) atomicAdd(&s_lvl[(k - a.q0) * nz2 + kc], q[k]);
+      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+      if (lane_id() == lead) atomicAdd(&a.lwp[col], v);
+      if (mine) col = -1;
+      todo = __ballot(col >= 0);
     }
-    if (first && c.ipt >= 1 && c.ipt <= a.g.nnx && c.jpt >= 1 && c.jpt <= a.g.nny)
-      atomicAdd(&a.lwp[(c.ipt - 1) + (int64_t)a.g.nnx * (c.jpt - 1)], m * mw);
+    if (col >= 0) atomicAdd(&a.lwp[col], water);
   }
   if (first) {
 #pragma unroll
@@ -1373,16 +1488,44 @@ __global__ void __launch_bounds__(kBlock) k_xy_stats(StatsArgs a) {
   for (int i = threadIdx.x; i < a.nq * nz2; i += blockDim.x) a.part1[(int64_t)blockIdx.x * a.nq * nz2 + i] = s_lvl[i];
 }
 
-// Sums (maxima, minima) of the workgroup rows in row order.
-__global__ void k_xy_reduce(const double* part, int rows, int width, double* out, int kind_split0, int kind_split1) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= width) return;
-  double v = part[i];
-  for (int r = 1; r < rows; ++r) {
-    const double w = part[(int64_t)r * width + i];
-    v = (i < kind_split0) ? v + w : (i < kind_split1 ? fmax(v, w) : fmin(v, w));
+// Sums (maxima, minima) of the workgroup rows: values `first` and up of the
+// whole-domain rows (kStats0 wide, part0) in the last workgroup, those of the
+// level rows (part1) in the others.  A workgroup takes 64 values, each wave a run of
+// rows/16 rows of them, and adds the waves' results in row order.  Bound by the
+// latency of the loads, so a wave keeps eight in flight; one thread for all
+// rows of a value took 68 us a launch for 256 rows.
+constexpr int kReduceWaves = 16;
+__global__ void __launch_bounds__(64 * kReduceWaves) k_xy_reduce(const double* part0, double* out0, const double* part1,
+                                                                 double* out1, int rows, int width1) {
+  __shared__ double s_part[kReduceWaves][64];
+  const bool whole = part0 && blockIdx.x == gridDim.x - 1;
+  const double* part = whole ? part0 : part1;
+  const int width = whole ? kStats0 : width1;
+  const int lane = lane_id(), wid = threadIdx.x >> 6;
+  const int i = whole ? lane : (int)blockIdx.x * 64 + lane;
+  const bool is_max = whole && i >= 9 && i < 15, is_min = whole && i >= 15;
+  auto fold = [&](double v, double w) { return is_max ? fmax(v, w) : is_min ? fmin(v, w) : v + w; };
+  const int per = (rows + kReduceWaves - 1) / kReduceWaves;
+  const int r0 = wid * per, r1 = min(rows, r0 + per);
+  if (i < width && r0 < r1) {
+    double v = part[(int64_t)r0 * width + i];
+    int r = r0 + 1;
+    for (; r + 8 <= r1; r += 8) {
+      double w[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w[k] = part[(int64_t)(r + k) * width + i];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v = fold(v, w[k]);
+    }
+    for (; r < r1; ++r) v = fold(v, part[(int64_t)r * width + i]);
+    s_part[wid][lane] = v;
   }
-  out[i] = v;
+  __syncthreads();
+  if (wid == 0 && i < width) {
+    double v = s_part[0][lane];
+    for (int w = 1; w * per < rows; ++w) v = fold(v, s_part[w][lane]);
+    (whole ? out0 : out1)[i] = v;
+  }
 }
 
 // Exclusive scan of the u-cell histogram: k_scan_reduce sums its tiles, then

@@ -508,6 +508,28 @@ int bin_current(int32_t* cellidx_dev, const int32_t* tie, bool canonical = true)
   return finish_bin(tie, canonical);
 }
 
+// the positions of the current slots, for the kernels that work out the cells
+BinArgs cell_args() {
+  BinArgs b{};
+  b.g = ctx.g;
+  b.hot = ctx.hot[ctx.cur];
+  b.n = ctx.n;
+  b.cap = ctx.cap;
+  return b;
+}
+
+// the droplets of a w cell as a run of the cell sort, made here if the last
+// step did not leave it (interleaved levels only)
+int wcell_args(WcellArgs& w) {
+  if (!ctx.perm_valid || !ctx.keys_valid) CHK(bin_current(nullptr, nullptr, false));
+  w.g = ctx.g;
+  w.hot = ctx.hot[ctx.cur];
+  w.mult = ctx.mult[ctx.cur];
+  w.perm = ctx.perm;
+  w.offsets = ctx.offsets;
+  return 0;
+}
+
 unsigned src_mask() {
   unsigned m = 0;
   if (ctx.fl.icouple == 1) m |= 7u;
@@ -710,13 +732,15 @@ int stats_scratch(double** ws) {
 }
 
 struct StatsShape {
-  int nz2, rows, nq_max;
+  int nz2, rows, threads, nq_max;
 };
 
 StatsShape stats_shape() {
   StatsShape sh;
   sh.nz2 = ctx.g.nnz + 2;
   sh.rows = (int)std::min<int64_t>(kStatsRowsMax, std::max<int64_t>(1, (ctx.n + kBlock - 1) / kBlock));
+  const int64_t chunk = (ctx.n + sh.rows - 1) / sh.rows;  // slots of a workgroup
+  sh.threads = (int)std::min<int64_t>(kStatsBlock, std::max<int64_t>(1, (chunk + kBlock - 1) / kBlock) * kBlock);
   sh.nq_max = std::max(1, std::min(24, kStatsWidthMax / sh.nz2));
   return sh;
 }
@@ -753,12 +777,13 @@ int stats_launch(const StatsShape& sh, const ColdView& cold, double* part0, doub
     const size_t lds = sizeof(double) * a.nq * sh.nz2;
     const int width = a.nq * sh.nz2;
     double* dst = out1 + (int64_t)q0 * sh.nz2;
-    CHK(go("xy_stats", [&] { k_xy_stats<<<sh.rows, kBlock, lds, ctx.stream>>>(a); }));
-    CHK(go("xy_stats", [&] {
-      k_xy_reduce<<<(width + kBlock - 1) / kBlock, kBlock, 0, ctx.stream>>>(part1, sh.rows, width, dst, width, width);
+    CHK(go("xy_stats", [&] { k_xy_stats<<<sh.rows, sh.threads, lds, ctx.stream>>>(a); }));
+    // the whole-domain rows after the first pass only
+    const double* whole = q0 == 0 ? part0 : nullptr;
+    const unsigned nb = (unsigned)((width + 63) / 64) + (whole ? 1 : 0);
+    CHK(go("xy_reduce", [&] {
+      k_xy_reduce<<<nb, 64 * kReduceWaves, 0, ctx.stream>>>(whole, out0, part1, dst, sh.rows, width);
     }));
-    if (q0 == 0)
-      CHK(go("xy_stats", [&] { k_xy_reduce<<<1, kBlock, 0, ctx.stream>>>(part0, sh.rows, kStats0, out0, 9, 15); }));
   }
   return 0;
 }
@@ -1721,25 +1746,21 @@ int ntlp_gpu_wcell_counts(int32_t* num_array) {
   CHK(need_init());
   if (!num_array) return fail(NTLP_E_INVALID, "null output");
   const int64_t nw = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
-  int32_t* d = nullptr;
-  CHK(dalloc(d, nw, "w-cell counts"));
-  int rc = fill_i32(d, nw, 0);
-  if (rc == 0 && ctx.n > 0) {
-    BinArgs b;
-    b.g = ctx.g;
-    b.hot = ctx.hot[ctx.cur];
-    b.n = ctx.n;
-    b.cap = ctx.cap;
-    b.keys = nullptr;
-    b.counts = nullptr;
-    b.cellidx = nullptr;
-    rc = launch("wcells", [&] { k_wcells<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(b, d); });
+  CHK(xfer_stage((nw + 1) / 2, (nw + 1) / 2));
+  int32_t* d = reinterpret_cast<int32_t*>(ctx.xfer);
+  if (ctx.n > 0 && ctx.g.interleaved) {
+    WcellArgs w;
+    CHK(wcell_args(w));
+    const int64_t nt = (int64_t)((ctx.g.nnx + kWcellI - 1) / kWcellI) * ((ctx.g.nnz + kWcellK - 1) / kWcellK) * ctx.g.nny;
+    CHK(launch("wcells", [&] { k_wcells_sorted<<<(unsigned)nt, kBlock, 0, ctx.stream>>>(w, d); }));
+  } else {
+    CHK(fill_i32(d, nw, 0));
+    const BinArgs b = cell_args();
+    if (ctx.n > 0) CHK(launch("wcells", [&] { k_wcells<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(b, d); }));
   }
-  if (rc == 0 && to_host(num_array, d, sizeof(int32_t) * nw) != 0)
-    rc = fail(NTLP_E_HIP, "copy failed");
-  if (hipStreamSynchronize(ctx.stream) != hipSuccess && rc == 0) rc = fail(NTLP_E_HIP, "sync failed");
-  dfree(d);
-  return rc;
+  CHK(to_host(num_array, d, sizeof(int32_t) * nw));
+  HIPCHK(hipStreamSynchronize(ctx.stream));
+  return NTLP_OK;
 }
 
 int ntlp_gpu_calc_tauc_min(double* tauc_min) {
@@ -1750,39 +1771,28 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
     return NTLP_OK;
   }
   const int64_t ncell = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
-  double *rad = nullptr, *nc = nullptr;
-  int32_t* num = nullptr;
-  unsigned long long* res = nullptr;
-  int rc = dalloc(rad, ncell, "tauc sums");
-  if (!rc) rc = dalloc(nc, ncell, "tauc sums");
-  if (!rc) rc = dalloc(num, ncell, "tauc counts");
-  if (!rc) rc = dalloc(res, 1, "tauc result");
-  const double start = 1.0e10;
-  if (!rc && (hipMemsetAsync(rad, 0, sizeof(double) * ncell, ctx.stream) != hipSuccess ||
-              hipMemsetAsync(nc, 0, sizeof(double) * ncell, ctx.stream) != hipSuccess ||
-              hipMemsetAsync(num, 0, sizeof(int32_t) * ncell, ctx.stream) != hipSuccess ||
-              to_device(res, &start, sizeof(double)) != 0))
-    rc = fail(NTLP_E_HIP, "tauc_min set-up failed");
-  if (!rc) {
-    BinArgs b;
-    b.g = ctx.g;
-    b.hot = ctx.hot[ctx.cur];
-    b.n = ctx.n;
-    b.cap = ctx.cap;
+  const bool runs = ctx.g.interleaved;
+  const int64_t room = runs ? 1 : 1 + 2 * ncell + (ncell + 1) / 2;
+  CHK(xfer_stage(room, room));
+  unsigned long long* res = reinterpret_cast<unsigned long long*>(ctx.xfer);
+  if (!runs) CHK(fill_f64(ctx.xfer, room, 0.0));
+  CHK(fill_f64(ctx.xfer, 1, 1.0e10));
+  if (runs) {
+    WcellArgs w;
+    CHK(wcell_args(w));
+    CHK(launch("tauc", [&] { k_tauc_sorted<<<grid_flat(ncell), kBlock, 0, ctx.stream>>>(w, ctx.C, res); }));
+  } else {
+    double* rad = ctx.xfer + 1;
+    double* nc = rad + ncell;
+    int32_t* num = reinterpret_cast<int32_t*>(nc + ncell);
+    const BinArgs b = cell_args();
     const int64_t* mult = ctx.mult[ctx.cur];
-    rc = launch("tauc", [&] { k_tauc_accum<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(b, mult, rad, num, nc); });
+    CHK(launch("tauc", [&] { k_tauc_accum<<<grid8(ctx.n), kBlock, 0, ctx.stream>>>(b, mult, rad, num, nc); }));
+    CHK(launch("tauc", [&] { k_tauc_min<<<grid_flat(ncell), kBlock, 0, ctx.stream>>>(ctx.g, ctx.C, rad, num, nc, res); }));
   }
-  if (!rc)
-    rc = launch("tauc", [&] { k_tauc_min<<<grid_flat(ncell), kBlock, 0, ctx.stream>>>(ctx.g, ctx.C, rad, num, nc, res); });
   double m = 0.0;
-  if (!rc && (to_host(&m, res, sizeof(double)) != 0 ||
-              hipStreamSynchronize(ctx.stream) != hipSuccess))
-    rc = fail(NTLP_E_HIP, "tauc_min failed");
-  dfree(rad);
-  dfree(nc);
-  dfree(num);
-  dfree(res);
-  if (rc) return rc;
+  CHK(to_host(&m, res, sizeof(double)));
+  HIPCHK(hipStreamSynchronize(ctx.stream));
   *tauc_min = m * 5.0;
   return NTLP_OK;
 }
@@ -1792,24 +1802,19 @@ int ntlp_gpu_particle_xy_stats(double* s0, double* s1, double* lwp) {
   ColdView cold;
   CHK(cold_view(kDiagStats, cold));
   const StatsShape sh = stats_shape();
-  double *part0 = nullptr, *part1 = nullptr, *out0 = nullptr, *out1 = nullptr, *lw = nullptr;
-  int rc = dalloc(part0, (int64_t)sh.rows * kStats0, "statistics rows");
-  if (!rc) rc = dalloc(part1, (int64_t)sh.rows * sh.nq_max * sh.nz2, "statistics rows");
-  if (!rc) rc = dalloc(out0, kStats0, "statistics");
-  if (!rc) rc = dalloc(out1, 24 * sh.nz2, "statistics");
-  if (!rc) rc = dalloc(lw, (int64_t)ctx.g.nnx * ctx.g.nny, "LWP");
-  if (!rc) rc = stats_launch(sh, cold, part0, part1, out0, out1, lw, true);
-  if (!rc && ((s0 && to_host(s0, out0, sizeof(double) * kStats0) != 0) ||
-              (s1 && to_host(s1, out1, sizeof(double) * 24 * sh.nz2) != 0) ||
-              (lwp && to_host(lwp, lw, sizeof(double) * ctx.g.nnx * ctx.g.nny) != 0) ||
-              hipStreamSynchronize(ctx.stream) != hipSuccess))
-    rc = fail(NTLP_E_HIP, "statistics copy failed");
-  dfree(part0);
-  dfree(part1);
-  dfree(out0);
-  dfree(out1);
-  dfree(lw);
-  return rc;
+  const int64_t nlw = (int64_t)ctx.g.nnx * ctx.g.nny, n0 = (int64_t)sh.rows * kStats0;
+  const int64_t n1 = (int64_t)sh.rows * sh.nq_max * sh.nz2;
+  const int64_t room = kStats0 + 24 * sh.nz2 + nlw + n0 + n1;
+  CHK(xfer_stage(room, room));
+  double* out0 = ctx.xfer;
+  double* out1 = out0 + kStats0;
+  double* lw = out1 + 24 * sh.nz2;
+  CHK(stats_launch(sh, cold, lw + nlw, lw + nlw + n0, out0, out1, lw, true));
+  if (s0) CHK(to_host(s0, out0, sizeof(double) * kStats0));
+  if (s1) CHK(to_host(s1, out1, sizeof(double) * 24 * sh.nz2));
+  if (lwp) CHK(to_host(lwp, lw, sizeof(double) * nlw));
+  HIPCHK(hipStreamSynchronize(ctx.stream));
+  return NTLP_OK;
 }
 
 int ntlp_gpu_particle_xy_stats_noalloc(double* s0, double* s1, double* lwp) {
