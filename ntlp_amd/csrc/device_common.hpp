@@ -58,6 +58,10 @@ struct DevConsts {
   // 0.6 Sc^(1/3), 0.6 Pra^(1/3) of Sherwood/Nusselt: read from the constants
   // (scalar registers) rather than kept per droplet in vector registers
   double sc6, pr6;
+  // div_ok: the constants lie in the range that the quotients through
+  // reciprocals are meant for
+  double irhow, iSc, iPra;
+  int div_ok, pad_;
 };
 
 struct DevFlags {

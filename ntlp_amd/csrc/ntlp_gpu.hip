@@ -432,6 +432,12 @@ void derive_consts(DevConsts& C) {
   C.isurf_rho = 1.0 / C.surf_rho;
   C.sc6 = 0.6 * C.Sc13;
   C.pr6 = 0.6 * C.Pra13;
+  C.irhow = 1.0 / C.rhow;
+  C.iSc = 1.0 / C.Sc;
+  C.iPra = 1.0 / C.Pra;
+  C.div_ok = 1;
+  for (const double b : {C.nuf, C.rhow, C.Sc, C.Pra, C.pi2, C.Mw, C.Ru, C.Mw2Gam, C.Ru_rhow, C.Cpp})
+    if (!(b >= 0x1p-40 && b <= 0x1p40)) C.div_ok = 0;
 }
 
 // the device copy of ctx.C, in stream order with the kernels that read it
