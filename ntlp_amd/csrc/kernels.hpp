@@ -425,7 +425,9 @@ __device__ __forceinline__ void count_key(int* counts, int key, bool valid) {
 // no coupling amounts are formed.
 // LAZY (BE steps of the library): the residence times stay in HBM until
 // k_res_settle at the end of the call.
-template <int MODE, int PREC, int ILIN, bool SERVE = false, bool LAZY = false>
+// KEEP: see lv_solver.
+template <int MODE, int PREC, int ILIN, bool SERVE = false, bool LAZY = false,
+          bool KEEP = SERVE || PREC != PREC_MIXED || ILIN != 1>
 __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
   const DevConsts& C = *a.Cp;
   extern __shared__ double s_dyn[];  // z(0:nnz+1) | zz(0:nnz+1) | field box (a.box_bytes)
@@ -476,9 +478,8 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
         rk3_droplet<PREC, ILIN>(a.g, C, a.fl, a.F, s_z, s_zz, d, st, a.it, o, o.kpt, &bx);
     } else {
       // q* is a diagnostic of the record: formed on the step that stores it
-      constexpr bool keep = SERVE || PREC != PREC_MIXED || ILIN != 1;  // see lv_solver
-      be_droplet<PREC, ILIN, LAZY, keep>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, kg, SERVE ? nullptr : a.flux,
-                                   mult, &bx, !SERVE && a.write_cold);
+      be_droplet<PREC, ILIN, LAZY, KEEP>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, kg, SERVE ? nullptr : a.flux,
+                                         mult, &bx, !SERVE && a.write_cold);
     }
     if (SERVE && a.serve->last[home >> kServeIdxBits]) {
       const int64_t row = a.serve->out_off[home >> kServeIdxBits] + (home & kServeIdxMask);

@@ -798,10 +798,25 @@ template <int PREC, int ILIN>
 void launch_update_t(const StepArgs& a, const ColdView& rhs, unsigned grid) {
   k_update<PREC, ILIN><<<grid, kBlock, 0, ctx.stream>>>(a, rhs);
 }
+// Mixed backward-Euler steps whose fallback solves keep what they evaluated (141
+// registers instead of 125): as long as all droplets are in flight at three waves on
+// each of 1024 SIMDs, there is nothing that a fourth wave would hold.  With 0.02 %
+// of the solves falling back, a step of 1000, 100k and 190k droplets takes 67, 106
+// and 108 us instead of 89, 157 and 152, without such solves the same (22, 27
+// and 31).  Above, the three waves cost steps without such solves 3 to 11 % (260k:
+// 38 us against 34, 6M: 482 against 428).
+constexpr int64_t kKeepMax = 3 * 1024 * 64;
 template <int MODE, int PREC, int ILIN>
 void launch_step_t(const StepArgs& a, unsigned grid, bool lazy) {
   const size_t lds = step_lds_bytes(a.g.nnz, a.box_bytes);
   if constexpr (MODE == 2) {
+    if constexpr (PREC == PREC_MIXED && ILIN == 1) {
+      if (a.n <= kKeepMax) {
+        if (lazy) k_step<MODE, PREC, ILIN, false, true, true><<<grid, kBlock, lds, ctx.stream>>>(a);
+        else k_step<MODE, PREC, ILIN, false, false, true><<<grid, kBlock, lds, ctx.stream>>>(a);
+        return;
+      }
+    }
     if (lazy) {
       k_step<MODE, PREC, ILIN, false, true><<<grid, kBlock, lds, ctx.stream>>>(a);
       return;

@@ -357,9 +357,9 @@ struct LmPoint {
 // Jacobian together: an accepted candidate's values are the next iteration's,
 // a rejected iteration keeps the old ones.  That halves the chain, for 16
 // registers (a burst of 16 served ensembles, 0.02 % of whose solves fall back:
-// 9.97 -> 9.01 ms); the mixed step of the library, at 123 of the 128 that four waves
-// per SIMD leave, evaluates again instead (KEEP false: 141 registers and three
-// waves cost more than the tail).
+// 9.97 -> 9.01 ms).  The mixed step of the library, at 123 of the 128 that four waves
+// per SIMD leave, evaluates again instead where it has more droplets than three
+// waves a SIMD hold (KEEP false; see kKeepMax).
 template <bool KEEP, class Ev>
 __device__ __forceinline__ int lv_solver(const Ev& ev, const double vec1[2], double vec2[2], int& iters) {
   int iterations = 0, flag = 0;
