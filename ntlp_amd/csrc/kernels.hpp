@@ -431,9 +431,10 @@ __device__ __forceinline__ void count_key(int* counts, int key, bool valid) {
 // no coupling amounts are formed.
 // LAZY (BE steps of the library): the residence times stay in HBM until
 // k_res_settle at the end of the call.
-// KEEP: see lv_solver.
-template <int MODE, int PREC, int ILIN, bool SERVE = false, bool LAZY = false,
-          bool KEEP = SERVE || PREC != PREC_MIXED || ILIN != 1>
+// MODE: 1 RK3, 2 backward Euler, 3 the mixed backward-Euler step of a population
+// that three waves a SIMD hold (kKeepMax), whose fallback solves keep what they
+// evaluated (lv_solver).
+template <int MODE, int PREC, int ILIN, bool SERVE = false, bool LAZY = false>
 __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
   const DevConsts& C = *a.Cp;
   extern __shared__ double s_dyn[];  // z(0:nnz+1) | zz(0:nnz+1) | field box (a.box_bytes)
@@ -447,7 +448,7 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
   Tally tl = {0, 0, 0, 0, 0, 0, 0, -1};
   int key = -1;
   const bool inplace = !SERVE && a.inplace;
-  static_assert(!LAZY || (MODE == 2 && !SERVE), "lazy residence times: library BE steps only");
+  static_assert(!LAZY || (MODE != 1 && !SERVE), "lazy residence times: library BE steps only");
   // the droplet's loads are issued before the levels and the field box are
   // staged (a barrier orders every memory access around it), so that they are
   // in flight while those load
@@ -484,7 +485,8 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
         rk3_droplet<PREC, ILIN>(a.g, C, a.fl, a.F, s_z, s_zz, d, st, a.it, o, o.kpt, &bx);
     } else {
       // q* is a diagnostic of the record: formed on the step that stores it
-      be_droplet<PREC, ILIN, LAZY, KEEP>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, kg, SERVE ? nullptr : a.flux,
+      constexpr bool keep = SERVE || PREC != PREC_MIXED || ILIN != 1 || MODE == 3;
+      be_droplet<PREC, ILIN, LAZY, keep>(a.g, C, a.fl, a.F, s_z, s_zz, d, a.it, o, tl, kg, SERVE ? nullptr : a.flux,
                                          mult, &bx, !SERVE && a.write_cold);
     }
     if (SERVE && a.serve->last[home >> kServeIdxBits]) {
@@ -532,7 +534,7 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_step(StepArgs a) {
     }
   }
   count_key(a.counts, key, valid);
-  if (MODE == 2) flush_tally(tl, a.tally, s_red);
+  if (MODE != 1) flush_tally(tl, a.tally, s_red);
 }
 
 // ------------------------------------------------- reference entry points

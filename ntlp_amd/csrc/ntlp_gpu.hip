@@ -812,8 +812,8 @@ void launch_step_t(const StepArgs& a, unsigned grid, bool lazy) {
   if constexpr (MODE == 2) {
     if constexpr (PREC == PREC_MIXED && ILIN == 1) {
       if (a.n <= kKeepMax) {
-        if (lazy) k_step<MODE, PREC, ILIN, false, true, true><<<grid, kBlock, lds, ctx.stream>>>(a);
-        else k_step<MODE, PREC, ILIN, false, false, true><<<grid, kBlock, lds, ctx.stream>>>(a);
+        if (lazy) k_step<3, PREC, ILIN, false, true><<<grid, kBlock, lds, ctx.stream>>>(a);
+        else k_step<3, PREC, ILIN><<<grid, kBlock, lds, ctx.stream>>>(a);
         return;
       }
     }
