@@ -1939,6 +1939,10 @@ struct GenArgs {
   DevConsts C;
   DevFlags fl;
   DevFields F;
+  // A single ensemble comes with the arguments (start null), more of them in
+  // device memory: generating 1000 droplets of one took 94 us with its upload and
+  // the buffers for it, 50 us so, 20M 4291 and 4025 (its constants in scalar registers).
+  DevEnsemble one;
   const DevEnsemble* ens;  // [nens]
   const int64_t* start;    // [nens + 1]: first droplet of each ensemble, then n
   int nens;
@@ -1967,6 +1971,18 @@ __device__ __forceinline__ int gen_ensemble(const GenArgs& a, int64_t i) {
   return lo;
 }
 
+// f(ensemble, index of droplet i in it)
+template <bool ONE, class F>
+__device__ __forceinline__ auto with_ensemble(const GenArgs& a, int64_t i, F f) {
+  if constexpr (ONE) {
+    return f(a.one, i);
+  } else {
+    const int en = gen_ensemble(a, i);
+    return f(a.ens[en], i - a.start[en]);
+  }
+}
+
+template <bool ONE>
 __global__ void __launch_bounds__(kBlock) k_gen_keys(GenArgs a) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   stage_grid(a.g, s_z, s_zz);
@@ -1975,20 +1991,19 @@ __global__ void __launch_bounds__(kBlock) k_gen_keys(GenArgs a) {
   const bool valid = i < a.n;
   int key = -1;
   if (valid) {
-    const int en = gen_ensemble(a, i);
-    const DevEnsemble& e = a.ens[en];
-    const int64_t k = i - a.start[en];
-    const NewDroplet nd = make_droplet(e, a.g, s_z, k, a.C.rhos, a.C.pi2);
+    const NewDroplet nd = with_ensemble<ONE>(a, i, [&](const DevEnsemble& e, int64_t k) {
+      a.pidx[i] = (int32_t)(e.first + k + 1);
+      return make_droplet(e, a.g, s_z, k, a.C.rhos, a.C.pi2);
+    });
     key = ukey_of(a.g, cell_of(a.g, s_z, s_zz, nd.x, nd.y, nd.z));
     a.put_keys[i] = key;
-    a.pidx[i] = (int32_t)(e.first + k + 1);
     a.procidx[i] = 0;
     for (int c = 0; c < kNCold; ++c) a.cold[(int64_t)c * a.cap + i] = 0.0;
   }
   count_key(a.counts, key, valid);
 }
 
-template <int ILIN>
+template <int ILIN, bool ONE>
 __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_generate(GenArgs a) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   stage_grid(a.g, s_z, s_zz);
@@ -1996,9 +2011,13 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_generate(GenArgs a)
   const int64_t t = xcd_block() * kBlock + threadIdx.x;
   if (t >= a.n) return;
   const int32_t i = a.perm[t];
-  const int en = gen_ensemble(a, i);
-  const DevEnsemble& e = a.ens[en];
-  const NewDroplet nd = make_droplet(e, a.g, s_z, i - a.start[en], a.C.rhos, a.C.pi2);
+  double kappa;
+  int64_t mult;
+  const NewDroplet nd = with_ensemble<ONE>(a, i, [&](const DevEnsemble& e, int64_t k) {
+    kappa = e.kappa_s;
+    mult = e.mult;
+    return make_droplet(e, a.g, s_z, k, a.C.rhos, a.C.pi2);
+  });
   const Cell c = cell_of(a.g, s_z, s_zz, nd.x, nd.y, nd.z);
   const Fluid f = (ILIN == 1) ? gather_lin_f64<true>(a.g, a.F, s_z, s_zz, nd.x, nd.y, nd.z, c)
                               : gather6_f64(a.g, a.F, s_z, s_zz, nd.x, nd.y, nd.z, c);
@@ -2012,11 +2031,11 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_generate(GenArgs a)
   d.Tp = f.T;
   d.r = nd.r;
   d.m_s = nd.m_s;
-  d.kappa = e.kappa_s;
-  d.rc = crit_radius_of(a.C, a.fl, nd.m_s, e.kappa_s, f.T);
+  d.kappa = kappa;
+  d.rc = crit_radius_of(a.C, a.fl, nd.m_s, kappa, f.T);
   d.res = d.actres = d.numact = 0.0;
   store_drop(a.hot, t, d);
-  a.mult[t] = e.mult;
+  a.mult[t] = mult;
   a.home[t] = i;
   a.keys[t] = ukey_of(a.g, c);
   a.diag[kCUFX * a.cap + t] = f.u[0];

@@ -440,6 +440,16 @@ void derive_consts(DevConsts& C) {
     if (!(b >= 0x1p-40 && b <= 0x1p40)) C.div_ok = 0;
 }
 
+// the critical-radius table of setup_radval (particles.f90:5294-5305), the same for
+// every context
+int upload_radval(hipStream_t stream) {
+  static double table[1024];
+  const double radstart = -8.0, radend = -3.0, dr = (radstart - radend) / 1024.0;
+  for (int i = 1; i <= 1024; ++i) table[i - 1] = std::pow(10.0, radstart - (double)(i - 1) * dr);
+  HIPCHK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_radval), table, sizeof(table), 0, hipMemcpyHostToDevice, stream));
+  return 0;
+}
+
 // the device copy of ctx.C, in stream order with the kernels that read it
 int upload_consts() {
   HIPCHK(hipMemcpyAsync(ctx.d_consts, &ctx.C, sizeof(DevConsts), hipMemcpyHostToDevice, ctx.stream));
@@ -1105,6 +1115,7 @@ int ntlp_gpu_init(const ntlp_grid* grid, const ntlp_consts* c, const ntlp_flags*
   ctx.ext_elems = (int64_t)(nz + 2) * (grid->nny + 5) * (grid->nnx + 5);
   ctx.init = true;
   CHK(upload_consts());
+  CHK(upload_radval(ctx.stream));
   CHK(fill_i32(ctx.counts, ctx.ncell, 0));
   CHK(fill_f64(ctx.src, 6 * ctx.nsrc, 0.0));
   CHK(launch("fill", [&] { k_fill_u64<<<64, kBlock, 0, ctx.stream>>>(ctx.tally, kTallyRows * kTallyWidth); }));
@@ -1201,15 +1212,6 @@ int ensure_capacity(int64_t n) {
   ctx.slots_sorted = false;
   ctx.perm_valid = false;
   ctx.keys_valid = false;
-  return 0;
-}
-
-// the critical-radius table of setup_radval (particles.f90:5294-5305)
-int upload_radval(hipStream_t stream) {
-  static double table[1024];
-  const double radstart = -8.0, radend = -3.0, dr = (radstart - radend) / 1024.0;
-  for (int i = 1; i <= 1024; ++i) table[i - 1] = std::pow(10.0, radstart - (double)(i - 1) * dr);
-  HIPCHK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_radval), table, sizeof(table), 0, hipMemcpyHostToDevice, stream));
   return 0;
 }
 
@@ -1471,19 +1473,23 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
   const int64_t n = start[nens];
   if (n < 1 || n >= (int64_t)INT32_MAX) return fail(NTLP_E_RANGE, "the ensembles must hold 1 .. 2^31-2 droplets");
   CHK(ensure_capacity(n));
-  CHK(upload_radval(ctx.stream));
   DevEnsemble* d_ens = nullptr;
   int64_t* d_start = nullptr;
-  CHK(dalloc(d_ens, nens, "ensembles"));
-  int rc = dalloc(d_start, nens + 1, "ensemble starts");
-  if (!rc && (to_device(d_ens, de.data(), sizeof(DevEnsemble) * nens) != 0 ||
-              to_device(d_start, start.data(), sizeof(int64_t) * (nens + 1)) != 0))
-    rc = fail(NTLP_E_HIP, "ensemble upload failed");
+  if (nens > 1) {
+    static_assert(sizeof(DevEnsemble) % 8 == 0, "whole words of the staging buffer");
+    const int64_t words = nens * (int64_t)(sizeof(DevEnsemble) / 8), room = words + nens + 1;
+    CHK(xfer_stage(room, room));
+    d_ens = reinterpret_cast<DevEnsemble*>(ctx.xfer);
+    d_start = reinterpret_cast<int64_t*>(ctx.xfer + words);
+    CHK(to_device(d_ens, de.data(), sizeof(DevEnsemble) * nens));
+    CHK(to_device(d_start, start.data(), sizeof(int64_t) * (nens + 1)));
+  }
   GenArgs a;
   a.g = ctx.g;
   a.C = ctx.C;
   a.fl = ctx.fl;
   a.F = fields_view();
+  a.one = de[0];
   a.ens = d_ens;
   a.start = d_start;
   a.nens = nens;
@@ -1502,12 +1508,18 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
   a.perm = ctx.perm;
   const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
   const bool lin = ctx.fl.ilin == 1;
-  if (!rc) rc = launch("generate", [&] { k_gen_keys<<<grid, kBlock, 0, ctx.stream>>>(a); });
+  const bool one = nens == 1;
+  int rc = launch("generate", [&] {
+    if (one) k_gen_keys<true><<<grid, kBlock, 0, ctx.stream>>>(a);
+    else k_gen_keys<false><<<grid, kBlock, 0, ctx.stream>>>(a);
+  });
   if (!rc) rc = sort_keys(ctx.keys[1], nullptr);
   if (!rc)
     rc = launch("generate", [&] {
-      if (lin) k_generate<1><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
-      else k_generate<0><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
+      if (lin && one) k_generate<1, true><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
+      else if (lin) k_generate<1, false><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
+      else if (one) k_generate<0, true><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
+      else k_generate<0, false><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
     });
   if (!rc) {  // slots in cell order with their keys; uf, Tf and qinf wait in diag
     ctx.home_identity = false;
@@ -1517,8 +1529,6 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
     ctx.diag_mask = kDiagFluid;
   }
   if (hipStreamSynchronize(ctx.stream) != hipSuccess && !rc) rc = fail(NTLP_E_HIP, "ensemble generation failed");
-  dfree(d_ens);
-  dfree(d_start);
   return rc;
 }
 
@@ -1547,7 +1557,6 @@ int ntlp_gpu_particles_get_column(int32_t column, double* out, int64_t n) {
 int ntlp_gpu_crit_radius(void) {
   CHK(need_init());
   if (ctx.n == 0) return NTLP_OK;
-  CHK(upload_radval(ctx.stream));
   StepArgs a = base_args();
   CHK(launch("crit_radius", [&] { k_crit_radius<<<grid_flat(ctx.n), kBlock, 0, ctx.stream>>>(a); }));
   HIPCHK(hipStreamSynchronize(ctx.stream));

@@ -624,7 +624,6 @@ int ntlp_serve_open(const ntlp_serve_config* cfg, int64_t* capacity) {
     HIPCHK(hipMemsetAsync(srv.tally, 0, sizeof(unsigned long long) * kTallySlots * kTallyWidth, srv.stream));
     HIPCHK(hipMemsetAsync(srv.keys[0], 0xff, sizeof(int32_t) * cap, srv.stream));
     HIPCHK(hipMemsetAsync(srv.keys[1], 0xff, sizeof(int32_t) * cap, srv.stream));
-    CHK(upload_radval(srv.stream));
     HIPCHK(hipStreamSynchronize(srv.stream));
     return 0;
   };
