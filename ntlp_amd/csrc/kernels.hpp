@@ -144,7 +144,7 @@ __device__ __forceinline__ long long wave_sum(long long v) {
 
 // Newton tallies are summed per workgroup (ballots and 32-bit wave sums, then
 // LDS) and added to one of kTallySlots counter slots, each on its own cache
-// lines, chosen by workgroup; k_tally_close folds the slots into the step's
+// lines, chosen by workgroup; close_tally folds the slots into the step's
 // row.  (One shared row would put every workgroup's atomics on one L2 line.)
 constexpr int kTallySlots = 64;
 
@@ -885,7 +885,7 @@ __global__ void __launch_bounds__(kBlock) k_scatter_pull(PullArgs a) {
 // and dealt to the threads kU droplets at a time: a thread first loads the
 // kU slots from perm, then the kU droplets' positions, keys and amounts, and
 // only then adds their in-box corners into LDS.  The kernel is bound by the
-// latency of those loads and by the FP64 LDS atomics, so it is kept small (67
+// latency of those loads and by the FP64 LDS atomics, so it is kept small (56
 // VGPRs, 25 KB of LDS) to keep six workgroups resident per CU.  The box is
 // finally stored with plain coalesced writes.  Every node belongs to exactly
 // one box, so the fields need no clearing.  A droplet near a box face is read
