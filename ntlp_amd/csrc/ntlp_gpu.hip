@@ -186,11 +186,27 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
+// Gives the kept staging buffer back (between the calls that use it); whether
+// there was one.
+bool drop_staging() {
+  if (!ctx.xfer) return false;
+  (void)hipStreamSynchronize(ctx.stream);
+  dfree(ctx.xfer);
+  ctx.xfer_cap = 0;
+  return true;
+}
+
+// Device memory; no call asks for any between xfer_stage and its use of it, so a
+// full device takes the staging buffer back first.
 template <typename T>
 int dalloc(T*& p, int64_t count, const char* what) {
   dfree(p);
   if (count <= 0) count = 1;
   hipError_t e = hipMalloc((void**)&p, sizeof(T) * (size_t)count);
+  if (e != hipSuccess && drop_staging()) {
+    (void)hipGetLastError();
+    e = hipMalloc((void**)&p, sizeof(T) * (size_t)count);
+  }
   if (e != hipSuccess) {
     p = nullptr;
     return fail(NTLP_E_NOMEM, std::string("hipMalloc failed for ") + what + " (" +
