@@ -23,6 +23,10 @@
  *    once, the coupling sources, counters and flux statistics are zero, and
  *    calc_tauc_min and the minima/maxima of particle_xy_stats keep the
  *    reference's start values.
+ *  - A call that replaces the droplets (put, put_records, read_part_res,
+ *    generate) and fails after its arguments were accepted leaves a context
+ *    without droplets: until they are put again, the calls that use them
+ *    return NTLP_E_STATE.
  *  - ntlp_gpu_init checks all its arguments before it touches the device, so
  *    a rejected call leaves an existing context as it was.
  */
@@ -41,7 +45,7 @@ extern "C" {
 #define NTLP_E_NOMEM (-4)       /* device allocation failed                  */
 #define NTLP_E_RANGE (-5)       /* size beyond a documented maximum          */
 #define NTLP_E_UNSUPPORTED (-6) /* flag combination the library does not run */
-#define NTLP_E_STATE (-7)       /* call out of order (no fields, a failed step) */
+#define NTLP_E_STATE (-7)       /* call out of order (no fields, a failed step or put) */
 
 /* Column order of the droplet real SoA block: column c of droplet i lives at
  * soa[c*n + i] (a Fortran array real(8) :: soa(n, NTLP_NREAL)).  These are

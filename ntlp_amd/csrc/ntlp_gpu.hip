@@ -203,11 +203,12 @@ int dalloc(T*& p, int64_t count, const char* what) {
   dfree(p);
   if (count <= 0) count = 1;
   hipError_t e = hipMalloc((void**)&p, sizeof(T) * (size_t)count);
-  if (e != hipSuccess && drop_staging()) {
-    (void)hipGetLastError();
-    e = hipMalloc((void**)&p, sizeof(T) * (size_t)count);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch would report it
+    if (drop_staging()) e = hipMalloc((void**)&p, sizeof(T) * (size_t)count);
   }
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     p = nullptr;
     return fail(NTLP_E_NOMEM, std::string("hipMalloc failed for ") + what + " (" +
                                   std::to_string(sizeof(T) * (size_t)count) + " bytes): " + hipGetErrorString(e));
@@ -281,7 +282,7 @@ int need_fields() {
 int need_drops() {
   CHK(need_fields());
   if (ctx.state_bad)
-    return fail(NTLP_E_STATE, "a failed step call left the droplets inconsistent: put them again");
+    return fail(NTLP_E_STATE, "a failed call left the droplets inconsistent: put them again");
   return 0;
 }
 
@@ -329,13 +330,11 @@ int to_host(void* dst, const void* src, size_t bytes) {
   return 0;
 }
 
-// The staging buffer with room for at least `least` doubles, `want` if that
-// stays below kXferBytes.  It is kept until the context is released: allocated
-// and freed on each call it cost 40 to 260 us.  Its users leave it to the next
-// in stream order.
-constexpr int64_t kXferBytes = 128ll << 20;
-int xfer_stage(int64_t least, int64_t want) {
-  const int64_t room = std::max(least, std::min<int64_t>(want, kXferBytes / 8));
+// The staging buffer with room for `room` doubles.  It is kept for the next
+// call, until the context is released or an allocation fails: allocated and
+// freed on each call it cost 40 to 260 us.  Its users leave it to the next in
+// stream order.
+int xfer_stage(int64_t room) {
   if (room <= ctx.xfer_cap) return 0;
   HIPCHK(hipStreamSynchronize(ctx.stream));
   ctx.xfer_cap = 0;
@@ -343,6 +342,36 @@ int xfer_stage(int64_t least, int64_t want) {
   ctx.xfer_cap = room;
   return 0;
 }
+
+// The device side of a droplet transfer: `want` doubles of the staging buffer;
+// where they are more than kXferBytes, or the device has no room for them, the
+// slots that no droplet stands in (hot[1 - cur]), so that droplets already on
+// the device can always be read back and a put needs no more memory than its
+// droplets.
+constexpr int64_t kXferBytes = 128ll << 20;
+struct Stage {
+  double* p;
+  int64_t room;  // doubles
+};
+Stage droplet_stage(int64_t want) {
+  if (want <= kXferBytes / 8 && xfer_stage(want) == 0) return {ctx.xfer, ctx.xfer_cap};
+  return {ctx.hot[1 - ctx.cur], tiled_elems(ctx.cap, kNHot)};
+}
+
+// Calls that replace the droplets: unless done() is reached, the context is
+// left without any, and asks for them again.
+struct Replacing {
+  bool complete = false;
+  int done() {
+    complete = true;
+    return NTLP_OK;
+  }
+  ~Replacing() {
+    if (complete) return;
+    ctx.n = 0;
+    ctx.state_bad = true;
+  }
+};
 
 void release_all() {
   for (auto& p : ctx.ext) dfree(p);
@@ -1175,7 +1204,7 @@ int ntlp_gpu_set_fields(const double* u, const double* v, const double* w, const
     if (!ctx.ext[f]) CHK(dalloc(ctx.ext[f], ctx.ext_elems, "ext field"));
   for (int f = 0; f < 3; ++f)
     if (!ctx.f32[f]) CHK(dalloc(ctx.f32[f], ctx.ext_elems, "fp32 field copy"));
-  if (layout != NTLP_LAYOUT_EXT) CHK(xfer_stage(in_elems, in_elems));
+  if (layout != NTLP_LAYOUT_EXT) CHK(xfer_stage(in_elems));
   // one staging buffer serves the fields in turn, in stream order
   for (int f = 0; f < 5; ++f) {
     double* dst = ctx.ext[f];
@@ -1203,6 +1232,7 @@ namespace {
 int ensure_capacity(int64_t n) {
   HIPCHK(hipStreamSynchronize(ctx.stream));
   if (n > ctx.cap) {
+    ctx.cap = 0;  // until all of them are there
     for (int b = 0; b < 2; ++b) {
       CHK(dalloc(ctx.hot[b], tiled_elems(n, kNHot), "hot state"));
       CHK(dalloc(ctx.mult[b], n, "mult"));
@@ -1273,17 +1303,18 @@ int ntlp_gpu_particles_put(const double* soa, const int64_t* mult, const int32_t
   CHK(need_init());
   if (n < 0 || (n > 0 && (!soa || !mult))) return fail(NTLP_E_INVALID, "bad droplet arrays");
   if (n >= (int64_t)INT32_MAX) return fail(NTLP_E_RANGE, "more than 2^31-1 droplets");
+  Replacing in;
   CHK(ensure_capacity(n));
-  if (n == 0) return NTLP_OK;
-  // as many columns at a time as the staging buffer holds
-  CHK(xfer_stage(n, NTLP_NREAL * n));
-  const int per = (int)std::min<int64_t>(NTLP_NREAL, ctx.xfer_cap / n);
+  if (n == 0) return in.done();
+  // as many columns at a time as the staging holds
+  const Stage st = droplet_stage(NTLP_NREAL * n);
+  const int per = (int)std::min<int64_t>(NTLP_NREAL, st.room / n);
   const ColumnPlace pl = column_places();
   for (int c = 0; c < NTLP_NREAL; c += per) {
     const int nc = std::min(per, NTLP_NREAL - c);
-    CHK(to_device(ctx.xfer, soa + (int64_t)c * n, sizeof(double) * nc * n));
+    CHK(to_device(st.p, soa + (int64_t)c * n, sizeof(double) * nc * n));
     CHK(launch("put", [&] {
-      k_columns_in<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(ctx.xfer, c, pl, n, ctx.cap,
+      k_columns_in<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(st.p, c, pl, n, ctx.cap,
                                                                                               ctx.hot[0], ctx.cold);
     }));
   }
@@ -1294,29 +1325,29 @@ int ntlp_gpu_particles_put(const double* soa, const int64_t* mult, const int32_t
   else CHK(fill_i32(ctx.procidx, n, 0));
   CHK(launch("iota", [&] { k_iota<<<grid_flat(n), kBlock, 0, ctx.stream>>>(ctx.home[0], n); }));
   HIPCHK(hipStreamSynchronize(ctx.stream));
-  return NTLP_OK;
+  return in.done();
 }
 
 int ntlp_gpu_particles_get(double* soa, int64_t* mult, int32_t* pidx, int32_t* procidx, int64_t n) {
   CHK(need_init());
   if (n != ctx.n) return fail(NTLP_E_INVALID, "n does not match the droplet count on the device");
   if (ctx.state_bad)
-    return fail(NTLP_E_STATE, "a failed step call left the droplets inconsistent: put them again");
+    return fail(NTLP_E_STATE, "a failed call left the droplets inconsistent: put them again");
   if (soa) CHK(flush_diag());
   if (n == 0) return NTLP_OK;
   const int32_t* home = ctx.home[ctx.cur];
   if (soa) {
-    CHK(xfer_stage(n, NTLP_NREAL * n));
-    const int per = (int)std::min<int64_t>(NTLP_NREAL, ctx.xfer_cap / n);
+    const Stage st = droplet_stage(NTLP_NREAL * n);
+    const int per = (int)std::min<int64_t>(NTLP_NREAL, st.room / n);
     const ColumnPlace pl = column_places();
     const int32_t* hm = ctx.home_identity ? nullptr : home;
     for (int c = 0; c < NTLP_NREAL; c += per) {
       const int nc = std::min(per, NTLP_NREAL - c);
       CHK(launch("get", [&] {
         k_columns_out<<<dim3((unsigned)((n + kBlock - 1) / kBlock), nc), kBlock, 0, ctx.stream>>>(
-            ctx.xfer, c, pl, n, ctx.cap, ctx.hot[ctx.cur], ctx.cold, hm);
+            st.p, c, pl, n, ctx.cap, ctx.hot[ctx.cur], ctx.cold, hm);
       }));
-      CHK(to_host(soa + (int64_t)c * n, ctx.xfer, sizeof(double) * nc * n));
+      CHK(to_host(soa + (int64_t)c * n, st.p, sizeof(double) * nc * n));
     }
   }
   if (mult) {
@@ -1364,34 +1395,35 @@ int ntlp_gpu_particles_put_records(const void* records, int64_t n) {
   if (n < 0 || (n > 0 && !records)) return fail(NTLP_E_INVALID, "bad record buffer");
   CHK(need_init());
   if (n >= (int64_t)INT32_MAX) return fail(NTLP_E_RANGE, "more than 2^31-1 droplets");
+  Replacing in;
   CHK(ensure_capacity(n));
-  if (n == 0) return NTLP_OK;
-  CHK(xfer_stage(kRecWords, kRecWords * n));
-  const int64_t per = std::min(n, ctx.xfer_cap / kRecWords);
+  if (n == 0) return in.done();
+  const Stage st = droplet_stage(kRecWords * n);
+  const int64_t per = std::min(n, st.room / kRecWords);
   const ColumnPlace pl = record_places();
   const unsigned char* base = (const unsigned char*)records;
   for (int64_t i = 0; i < n; i += per) {
     const int64_t m = std::min(per, n - i);
-    CHK(to_device(ctx.xfer, base + i * NTLP_RECORD_BYTES, (size_t)m * NTLP_RECORD_BYTES));
+    CHK(to_device(st.p, base + i * NTLP_RECORD_BYTES, (size_t)m * NTLP_RECORD_BYTES));
     CHK(launch("put", [&] {
       k_records_in<<<(unsigned)((m + kRecTile - 1) / kRecTile), kBlock, 0, ctx.stream>>>(
-          (const uint64_t*)ctx.xfer, i, m, pl, ctx.cap, ctx.hot[0], ctx.cold, ctx.mult[0], ctx.pidx, ctx.procidx);
+          (const uint64_t*)st.p, i, m, pl, ctx.cap, ctx.hot[0], ctx.cold, ctx.mult[0], ctx.pidx, ctx.procidx);
     }));
   }
   CHK(launch("iota", [&] { k_iota<<<grid_flat(n), kBlock, 0, ctx.stream>>>(ctx.home[0], n); }));
   HIPCHK(hipStreamSynchronize(ctx.stream));
-  return NTLP_OK;
+  return in.done();
 }
 
 int ntlp_gpu_particles_get_records(void* records, int64_t n) {
   CHK(need_init());
   if (n != ctx.n || (n > 0 && !records)) return fail(NTLP_E_INVALID, "bad record buffer");
   if (ctx.state_bad)
-    return fail(NTLP_E_STATE, "a failed step call left the droplets inconsistent: put them again");
+    return fail(NTLP_E_STATE, "a failed call left the droplets inconsistent: put them again");
   CHK(flush_diag());
   if (n == 0) return NTLP_OK;
-  CHK(xfer_stage(kRecWords, kRecWords * n));
-  const int64_t per = std::min(n, ctx.xfer_cap / kRecWords);
+  const Stage st = droplet_stage(kRecWords * n);
+  const int64_t per = std::min(n, st.room / kRecWords);
   const ColumnPlace pl = record_places();
   const int32_t* slot = nullptr;
   if (!ctx.home_identity) {  // put index -> slot
@@ -1404,9 +1436,9 @@ int ntlp_gpu_particles_get_records(void* records, int64_t n) {
     const int64_t m = std::min(per, n - i);
     CHK(launch("get", [&] {
       k_records_out<<<(unsigned)((m + kRecTile - 1) / kRecTile), kBlock, 0, ctx.stream>>>(
-          (uint64_t*)ctx.xfer, i, m, pl, ctx.cap, ctx.hot[ctx.cur], ctx.cold, ctx.mult[ctx.cur], ctx.pidx, ctx.procidx, slot);
+          (uint64_t*)st.p, i, m, pl, ctx.cap, ctx.hot[ctx.cur], ctx.cold, ctx.mult[ctx.cur], ctx.pidx, ctx.procidx, slot);
     }));
-    CHK(to_host(base + i * NTLP_RECORD_BYTES, ctx.xfer, (size_t)m * NTLP_RECORD_BYTES));
+    CHK(to_host(base + i * NTLP_RECORD_BYTES, st.p, (size_t)m * NTLP_RECORD_BYTES));
   }
   HIPCHK(hipStreamSynchronize(ctx.stream));
   return NTLP_OK;
@@ -1488,15 +1520,17 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
   }
   const int64_t n = start[nens];
   if (n < 1 || n >= (int64_t)INT32_MAX) return fail(NTLP_E_RANGE, "the ensembles must hold 1 .. 2^31-2 droplets");
+  Replacing in;
   CHK(ensure_capacity(n));
   DevEnsemble* d_ens = nullptr;
   int64_t* d_start = nullptr;
   if (nens > 1) {
     static_assert(sizeof(DevEnsemble) % 8 == 0, "whole words of the staging buffer");
     const int64_t words = nens * (int64_t)(sizeof(DevEnsemble) / 8), room = words + nens + 1;
-    CHK(xfer_stage(room, room));
-    d_ens = reinterpret_cast<DevEnsemble*>(ctx.xfer);
-    d_start = reinterpret_cast<int64_t*>(ctx.xfer + words);
+    const Stage st = droplet_stage(room);
+    if (st.room < room) return fail(NTLP_E_NOMEM, "no device memory for the ensembles");
+    d_ens = reinterpret_cast<DevEnsemble*>(st.p);
+    d_start = reinterpret_cast<int64_t*>(st.p + words);
     CHK(to_device(d_ens, de.data(), sizeof(DevEnsemble) * nens));
     CHK(to_device(d_start, start.data(), sizeof(int64_t) * (nens + 1)));
   }
@@ -1545,7 +1579,7 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
     ctx.diag_mask = kDiagFluid;
   }
   if (hipStreamSynchronize(ctx.stream) != hipSuccess && !rc) rc = fail(NTLP_E_HIP, "ensemble generation failed");
-  return rc;
+  return rc ? rc : in.done();
 }
 
 int ntlp_gpu_particles_get_column(int32_t column, double* out, int64_t n) {
@@ -1553,7 +1587,7 @@ int ntlp_gpu_particles_get_column(int32_t column, double* out, int64_t n) {
   if (n != ctx.n || !out) return fail(NTLP_E_INVALID, "n does not match the droplet count, or null output");
   if (column < 0 || column >= NTLP_NREAL) return fail(NTLP_E_INVALID, "unknown column");
   if (ctx.state_bad)
-    return fail(NTLP_E_STATE, "a failed step call left the droplets inconsistent: put them again");
+    return fail(NTLP_E_STATE, "a failed call left the droplets inconsistent: put them again");
   if (n == 0) return NTLP_OK;
   if (hot_of(column) >= 0) {
     const double* hot = ctx.hot[ctx.cur];
@@ -1699,7 +1733,7 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
     return fail(NTLP_E_INVALID, "apply_particle_coupling takes x-pencil or core arrays");
   const int nx = ctx.g.nnx, ny = ctx.g.nny, nz = ctx.g.nnz;
   const int64_t elems = layout == NTLP_LAYOUT_XPENCIL ? (int64_t)(nx + 2) * ny * (nz + 2) : (int64_t)(nz + 2) * ny * nx;
-  int rc = xfer_stage(2 * elems, 2 * elems);
+  int rc = xfer_stage(2 * elems);
   double* stage[2] = {ctx.xfer, ctx.xfer + elems};
   double* host[2] = {T, q};
   for (int i = 0; i < 2 && !rc; ++i)
@@ -1792,7 +1826,7 @@ int ntlp_gpu_wcell_counts(int32_t* num_array) {
   CHK(need_init());
   if (!num_array) return fail(NTLP_E_INVALID, "null output");
   const int64_t nw = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
-  CHK(xfer_stage((nw + 1) / 2, (nw + 1) / 2));
+  CHK(xfer_stage((nw + 1) / 2));
   int32_t* d = reinterpret_cast<int32_t*>(ctx.xfer);
   if (ctx.n > 0 && ctx.g.interleaved) {
     WcellArgs w;
@@ -1819,7 +1853,7 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
   const int64_t ncell = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
   const bool runs = ctx.g.interleaved;
   const int64_t room = runs ? 1 : 1 + 2 * ncell + (ncell + 1) / 2;
-  CHK(xfer_stage(room, room));
+  CHK(xfer_stage(room));
   unsigned long long* res = reinterpret_cast<unsigned long long*>(ctx.xfer);
   if (!runs) CHK(fill_f64(ctx.xfer, room, 0.0));
   CHK(fill_f64(ctx.xfer, 1, 1.0e10));
@@ -1851,7 +1885,7 @@ int ntlp_gpu_particle_xy_stats(double* s0, double* s1, double* lwp) {
   const int64_t nlw = (int64_t)ctx.g.nnx * ctx.g.nny, n0 = (int64_t)sh.rows * kStats0;
   const int64_t n1 = (int64_t)sh.rows * sh.nq_max * sh.nz2;
   const int64_t room = kStats0 + 24 * sh.nz2 + nlw + n0 + n1;
-  CHK(xfer_stage(room, room));
+  CHK(xfer_stage(room));
   double* out0 = ctx.xfer;
   double* out1 = out0 + kStats0;
   double* lw = out1 + 24 * sh.nz2;
