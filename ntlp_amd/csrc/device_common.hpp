@@ -644,7 +644,7 @@ __device__ __forceinline__ Fluid gather6_f64(const DevGrid& g, const DevFields& 
   {
     int lo = 0, hi = 5;
     if (c.kwpt == 0) { lo = 2; hi = 3; kw[0] = 1; kw[1] = 1; }
-    else if (c.kwpt < 0) { hi = -1; kw[0] = 1; kw[1] = 1; kw[2] = 1; }
+    else if (c.kwpt < 0) { hi = -1; kw[0] = 0; kw[1] = 0; kw[2] = 0; }  // among the other three
     else if (c.kwpt == 1) { lo = 1; hi = 4; kw[0] = 1; }
     else if (c.kwpt == nnz - 1) { lo = 2; hi = 3; kw[4] = nnz; kw[5] = nnz; }
     else if (c.kwpt >= nnz) { hi = -1; kw[2] = nnz; kw[3] = nnz; kw[4] = nnz; kw[5] = nnz; }
@@ -677,9 +677,13 @@ __device__ __forceinline__ Fluid gather6_f64(const DevGrid& g, const DevFields& 
   };
   // Two of the six levels as b and b + 1.  Where the lists above repeat a level
   // or step back, at most one of the entries that share a level has a weight,
-  // and levels further apart have none, so the weights move to their level.
+  // and levels further apart have none, so the weights move to their level.  No
+  // level is read that is not in the list (a NaN or an infinity there would pass
+  // through its zero weight): below a repeated nnz stands nnz - 1, above a repeated
+  // 0 or 1 the next level.
   auto pair_of = [&](const int k[6], const double w[6], double& w0, double& w1) {
-    const int a = clampi(k[0], 0, nnz + 1), d = clampi(k[1], 0, nnz + 1), b = min(min(a, d), nnz);
+    const int a = clampi(k[0], 0, nnz + 1), d = clampi(k[1], 0, nnz + 1);
+    const int b = min(min(a, d), a == d && a == nnz ? nnz - 1 : nnz);
     w0 = (a == b ? w[0] : 0.0) + (d == b ? w[1] : 0.0);
     w1 = (a != b ? w[0] : 0.0) + (d != b ? w[1] : 0.0);
     return (unsigned)b;
