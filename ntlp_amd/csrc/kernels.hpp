@@ -1227,6 +1227,14 @@ __global__ void __launch_bounds__(kBlock) k_keys(BinArgs a) {
 // holds them in one run of slots: every w cell looks through its run, without
 // atomics or a cleared array.  Slots of a first or last column (keys clamped
 // into the box) are checked for their own column as well.
+// Bound by the latency of the run's loads (offsets, perm, z), so the lanes that
+// share a run follow the mean number of droplets in a cell (wcell_lanes), and a
+// run that is long for them, in a cluster of droplets, is shared by the whole
+// wave.  Counts and tauc, us, against an atomic (three) for each droplet and
+// against one lane for each run, however long:
+//   128^3, 3M (1.4 a cell)            33 and  64; atomics  123 and  479; one lane   65 and    59
+//   24x20x16, 4M (520 a cell)        108 and  58; atomics  376 and  939; one lane 5284 and  1762
+//   128^3, 1M, a tenth in one cell   828 and 1400; atomics 1140 and 1434; one lane 28945 and 48172
 struct WcellArgs {
   DevGrid g;
   const double* hot;
@@ -1235,50 +1243,110 @@ struct WcellArgs {
   const int32_t* offsets;  // u-cell offsets of the sort
 };
 
-// f(slot) for every droplet of the w cell (i, j, kc): 0-based i and j, 1-based kc
-template <class F>
-__device__ __forceinline__ void each_of_wcell(const WcellArgs& a, const double* s_z, int i, int j, int kc, F f) {
-  const int key = kc - 1 + (a.g.nnz + 1) * (j + (a.g.nny + 1) * i);
-  const int b = a.offsets[key], e = a.offsets[key + 2];
+struct WcellSum {
+  int32_t num;
+  double rad, nc;
+};
+
+// positions b, b + stride, ... of the sort, up to e, of the w cell (i, j, kc):
+// 0-based i and j, 1-based kc.  Four positions at a time, so that their loads
+// (perm, then z) are in flight together.
+template <bool COUNT>
+__device__ __forceinline__ void add_run(const WcellArgs& a, const double* s_z, int i, int j, int kc, unsigned b, unsigned e,
+                                        unsigned stride, WcellSum& s) {
   const double lo = s_z[kc - 1], hi = s_z[kc];
   const bool edge = i == 0 || j == 0;
-  for (int p = b; p < e; ++p) {
-    const int64_t t = a.perm[p];
-    const double z = a.hot[hix(kHZ, t)];
-    if (!(hi > z) || lo > z) continue;  // first_gt(z) is another level
-    if (edge && ((int)floor(a.hot[hix(kHX, t)] / a.g.dx) != i || (int)floor(a.hot[hix(kHY, t)] / a.g.dy) != j)) continue;
-    f(t);
+  for (unsigned p = b; p < e; p += 4 * stride) {
+    int32_t t[4];
+    double z[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) t[u] = p + u * stride < e ? a.perm[p + u * stride] : -1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) z[u] = t[u] >= 0 ? a.hot[hix(kHZ, t[u])] : hi;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (!(hi > z[u]) || lo > z[u]) continue;  // first_gt(z) is another level
+      if (edge && ((int)floor(a.hot[hix(kHX, t[u])] / a.g.dx) != i || (int)floor(a.hot[hix(kHY, t[u])] / a.g.dy) != j)) continue;
+      ++s.num;
+      if (!COUNT) {
+        s.rad += a.hot[hix(kHR, t[u])];
+        s.nc += (double)a.mult[t[u]];
+      }
+    }
   }
 }
 
-// Bound by the latency of the run's loads (offsets, perm, z): a workgroup takes
-// kWcellI x kWcellK cells of one (j) row, levels along the lanes, where the
-// offsets and the runs are consecutive, and turns them in LDS so that the
-// counts leave in 128-byte pieces along i.  3M droplets on 128^3: 121 us
-// with an atomic for each droplet, 62 us so.
+template <bool COUNT>
+__device__ __forceinline__ void sum_lanes(WcellSum& s, int lanes) {
+  for (int o = lanes >> 1; o > 0; o >>= 1) {
+    s.num += __shfl_xor(s.num, o, 64);
+    if (!COUNT) {
+      s.rad += __shfl_xor(s.rad, o, 64);
+      s.nc += __shfl_xor(s.nc, o, 64);
+    }
+  }
+}
+
+// The droplets of a w cell, by `lanes` (a power of two) neighbouring lanes with
+// the same cell; every lane of the wave takes part (valid: it has a cell), and
+// every lane of the group gets the sums.  Lanes are few where cells are sparse,
+// so that many cells are under way; a run that is long for them is shared by
+// the whole wave, one after the other.
+constexpr unsigned kRunLong = 32;  // positions for each lane
+template <bool COUNT>
+__device__ __forceinline__ WcellSum wcell_sum(const WcellArgs& a, const double* s_z, bool valid, int i, int j, int kc,
+                                              int lanes) {
+  const int lane = lane_id(), sub = lane & (lanes - 1);
+  unsigned b = 0, e = 0;
+  if (valid) {
+    const int key = kc - 1 + (a.g.nnz + 1) * (j + (a.g.nny + 1) * i);
+    b = (unsigned)a.offsets[key];
+    e = (unsigned)a.offsets[key + 2];
+  }
+  const bool wide = lanes < 64 && e - b > kRunLong * lanes;
+  WcellSum s = {0, 0.0, 0.0};
+  if (!wide) add_run<COUNT>(a, s_z, valid ? i : 1, valid ? j : 1, valid ? kc : 1, b + sub, e, lanes, s);
+  sum_lanes<COUNT>(s, lanes);
+  unsigned long long todo = __ballot(wide && sub == 0);
+  while (todo) {
+    const int l = __ffsll((long long)todo) - 1;
+    todo &= todo - 1;
+    WcellSum w = {0, 0.0, 0.0};
+    add_run<COUNT>(a, s_z, __shfl(i, l, 64), __shfl(j, l, 64), __shfl(kc, l, 64), __shfl(b, l, 64) + lane,
+                   __shfl(e, l, 64), 64, w);
+    sum_lanes<COUNT>(w, 64);
+    if (lane - sub == l) s = w;
+  }
+  return s;
+}
+
+// A workgroup takes kWcellI columns by nk levels (a power of two) of one j row,
+// levels along the lanes, where the offsets and the runs are consecutive, and
+// turns the counts in LDS so that they leave in 128-byte pieces along i.
 constexpr int kWcellI = 32, kWcellK = 64;
-__global__ void __launch_bounds__(kBlock) k_wcells_sorted(WcellArgs a, int32_t* num) {
+__global__ void __launch_bounds__(kBlock) k_wcells_sorted(WcellArgs a, int lanes, int nk, int32_t* num) {
   __shared__ double s_z[kMaxLevels];
   __shared__ int32_t s_num[kWcellI][kWcellK + 1];
   for (int k = threadIdx.x; k < a.g.nnz + 2; k += blockDim.x) s_z[k] = a.g.z[k];
   __syncthreads();
-  const int nti = (a.g.nnx + kWcellI - 1) / kWcellI, ntk = (a.g.nnz + kWcellK - 1) / kWcellK;
-  const int i0 = (int)(blockIdx.x % nti) * kWcellI, k0 = (int)(blockIdx.x / nti % ntk) * kWcellK;
+  const int nti = (a.g.nnx + kWcellI - 1) / kWcellI, ntk = (a.g.nnz + nk - 1) / nk;
+  const int i0 = (int)(blockIdx.x % nti) * kWcellI, k0 = (int)(blockIdx.x / nti % ntk) * nk;
   const int j = (int)(blockIdx.x / nti / ntk);
-  const int kk = threadIdx.x % kWcellK;
-  for (int ii = threadIdx.x / kWcellK; ii < kWcellI; ii += kBlock / kWcellK) {
-    int c = 0;
-    if (i0 + ii < a.g.nnx && k0 + kk < a.g.nnz) each_of_wcell(a, s_z, i0 + ii, j, k0 + kk + 1, [&](int64_t) { ++c; });
-    s_num[ii][kk] = c;
+  const int cells = kWcellI * nk, step = kBlock / lanes;
+  for (int c0 = 0; c0 < cells; c0 += step) {
+    const int c = c0 + threadIdx.x / lanes, kk = c & (nk - 1), ii = c / nk;
+    const bool valid = c < cells && i0 + ii < a.g.nnx && k0 + kk < a.g.nnz;
+    const WcellSum s = wcell_sum<true>(a, s_z, valid, i0 + ii, j, k0 + kk + 1, lanes);
+    if (valid && (threadIdx.x & (lanes - 1)) == 0) s_num[ii][kk] = s.num;
   }
   __syncthreads();
   const int io = threadIdx.x % kWcellI;
-  for (int ko = threadIdx.x / kWcellI; ko < kWcellK; ko += kBlock / kWcellI)
+  for (int ko = threadIdx.x / kWcellI; ko < nk; ko += kBlock / kWcellI)
     if (i0 + io < a.g.nnx && k0 + ko < a.g.nnz)
       num[(i0 + io) + (int64_t)a.g.nnx * (j + (int64_t)a.g.nny * (k0 + ko))] = s_num[io][ko];
 }
 
-// The same for any grid: an atomic for each droplet.
+// The same for any grid and any order of the slots: an atomic for each droplet.
 __global__ void __launch_bounds__(kBlock) k_wcells(BinArgs a, int32_t* num) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
   stage_grid(a.g, s_z, s_zz);
@@ -1294,9 +1362,9 @@ __global__ void __launch_bounds__(kBlock) k_wcells(BinArgs a, int32_t* num) {
 
 // ------------------------------------------------------------ statistics
 
-// calc_tauc_min (particles.f90:3310-3368), over any grid, first half: radius sum, count and
-// multiplicity sum per w cell (ipt, jpt, kc); droplets outside (1:nnx,
-// 1:nny, 1:nnz) are not counted.
+// calc_tauc_min (particles.f90:3310-3368), over any grid and any order of the
+// slots, first half: radius sum, count and multiplicity sum per w cell (ipt, jpt,
+// kc); droplets outside (1:nnx, 1:nny, 1:nnz) are not counted.
 __global__ void __launch_bounds__(kBlock) k_tauc_accum(BinArgs a, const int64_t* mult, double* rad, int32_t* num,
                                                        double* nc) {
   __shared__ double s_z[kMaxLevels], s_zz[kMaxLevels];
@@ -1347,26 +1415,19 @@ __global__ void __launch_bounds__(kBlock) k_tauc_min(DevGrid g, DevConsts C, con
 }
 
 // Both halves at once where a w cell's droplets are one run of the sort: no
-// cell arrays to clear, to add to and to read back.  Levels along the lanes;
-// bound by the latency of the run's loads.  3M droplets on 128^3: 480 us
-// with three atomics for each droplet, 63 us so.
-__global__ void __launch_bounds__(kBlock) k_tauc_sorted(WcellArgs a, DevConsts C, unsigned long long* out) {
+// cell arrays to clear, to add to and to read back.  Levels along the lanes.
+__global__ void __launch_bounds__(kBlock) k_tauc_sorted(WcellArgs a, DevConsts C, int lanes, unsigned long long* out) {
   __shared__ double s_z[kMaxLevels];
   for (int k = threadIdx.x; k < a.g.nnz + 2; k += blockDim.x) s_z[k] = a.g.z[k];
   __syncthreads();
   const int64_t ncell = (int64_t)a.g.nnx * a.g.nny * a.g.nnz;
+  const int step = kBlock / lanes;
   double m = 1.0e10;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ncell; e += (int64_t)gridDim.x * blockDim.x) {
-    const int kc = (int)(e % a.g.nnz) + 1;
-    const int col = (int)(e / a.g.nnz);
-    double rad = 0.0, nc = 0.0;
-    int32_t num = 0;
-    each_of_wcell(a, s_z, col / a.g.nny, col % a.g.nny, kc, [&](int64_t t) {
-      rad += a.hot[hix(kHR, t)];
-      nc += (double)a.mult[t];
-      ++num;
-    });
-    if (num != 0) m = fmin(m, tauc_of(a.g, C, kc, rad, num, nc));
+  for (int64_t c0 = (int64_t)blockIdx.x * step; c0 < ncell; c0 += (int64_t)gridDim.x * step) {
+    const int64_t e = c0 + threadIdx.x / lanes;
+    const int kc = (int)(e % a.g.nnz) + 1, col = (int)(e / a.g.nnz);
+    const WcellSum s = wcell_sum<false>(a, s_z, e < ncell, col / a.g.nny, col % a.g.nny, kc, lanes);
+    if (s.num != 0) m = fmin(m, tauc_of(a.g, C, kc, s.rad, s.num, s.nc));
   }
   tauc_close(m, out);
 }

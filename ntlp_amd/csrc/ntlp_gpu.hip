@@ -591,6 +591,35 @@ int wcell_args(WcellArgs& w) {
   return 0;
 }
 
+// Lanes for each w cell: as many as leave each about kWcellVisits droplets, or
+// half of it, to look at (a cell's run holds those of two u cells).  A lane's
+// loads come four at a time, so fewer visits gain nothing, and more lanes leave
+// fewer cells under way.  tauc, us, with 1, 2, 4, 8, 16, 32, 64 lanes: 2.4 droplets a
+// cell on 256x256x128 303, 359, 522, ...; 9.5 on 128^3 456, 286, 243, 305, ...; 15 on
+// 64^3 164, 97, 56, 54, 71, ...; 39 on 24x20x16 133, 87, 25, 17, 14, 14, 16.
+constexpr int64_t kWcellVisits = 6;
+int wcell_lanes() {
+  const int64_t ncell = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
+  int lanes = 1;
+  while (lanes < 64 && 2 * ctx.n > kWcellVisits * lanes * ncell) lanes *= 2;
+  return lanes;
+}
+// Whether the cell queries go by runs of the cell sort or by an atomic (three)
+// for each droplet.  The sort is there after a step or a coupling update, and
+// quickly made where the slots stand in cell order; for slots in put order it
+// takes longer than the atomics.  Both queries after a put, atomics and sort:
+// 4M droplets on 64^3 301 + 575 and 710 + 303 us, on 128^3 525 + 615 and 855 +
+// 294, 42k on 128^3 287 + 81 and 302 + 67; a tenth of 1M in one cell 1.5 + 1.5 and
+// 3.4 + 1.5 ms.
+bool wcell_runs() {
+  return ctx.g.interleaved  // or a w cell's droplets are no run
+         && (ctx.slots_sorted || (ctx.perm_valid && ctx.keys_valid));
+}
+// Tiles of the count are made smaller while there are fewer, since each takes
+// its cells in turn: 128^3 with 3M droplets 56, 54 and 33 us with 256, 1024 and
+// 4096 tiles.
+constexpr int64_t kWcellTiles = 4096;
+
 unsigned src_mask() {
   unsigned m = 0;
   if (ctx.fl.icouple == 1) m |= 7u;
@@ -1828,11 +1857,14 @@ int ntlp_gpu_wcell_counts(int32_t* num_array) {
   const int64_t nw = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
   CHK(xfer_stage((nw + 1) / 2));
   int32_t* d = reinterpret_cast<int32_t*>(ctx.xfer);
-  if (ctx.n > 0 && ctx.g.interleaved) {
+  if (ctx.n > 0 && wcell_runs()) {
     WcellArgs w;
     CHK(wcell_args(w));
-    const int64_t nt = (int64_t)((ctx.g.nnx + kWcellI - 1) / kWcellI) * ((ctx.g.nnz + kWcellK - 1) / kWcellK) * ctx.g.nny;
-    CHK(launch("wcells", [&] { k_wcells_sorted<<<(unsigned)nt, kBlock, 0, ctx.stream>>>(w, d); }));
+    const int lanes = wcell_lanes();
+    int nk = kWcellK / lanes;
+    auto tiles = [&] { return (int64_t)((ctx.g.nnx + kWcellI - 1) / kWcellI) * ((ctx.g.nnz + nk - 1) / nk) * ctx.g.nny; };
+    while (tiles() < kWcellTiles && nk > 1 && nk * lanes > kBlock / kWcellI) nk /= 2;
+    CHK(launch("wcells", [&] { k_wcells_sorted<<<(unsigned)tiles(), kBlock, 0, ctx.stream>>>(w, lanes, nk, d); }));
   } else {
     CHK(fill_i32(d, nw, 0));
     const BinArgs b = cell_args();
@@ -1851,7 +1883,7 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
     return NTLP_OK;
   }
   const int64_t ncell = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
-  const bool runs = ctx.g.interleaved;
+  const bool runs = wcell_runs();
   const int64_t room = runs ? 1 : 1 + 2 * ncell + (ncell + 1) / 2;
   CHK(xfer_stage(room));
   unsigned long long* res = reinterpret_cast<unsigned long long*>(ctx.xfer);
@@ -1860,7 +1892,8 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
   if (runs) {
     WcellArgs w;
     CHK(wcell_args(w));
-    CHK(launch("tauc", [&] { k_tauc_sorted<<<grid_flat(ncell), kBlock, 0, ctx.stream>>>(w, ctx.C, res); }));
+    const int lanes = wcell_lanes();
+    CHK(launch("tauc", [&] { k_tauc_sorted<<<grid_flat(ncell * lanes), kBlock, 0, ctx.stream>>>(w, ctx.C, lanes, res); }));
   } else {
     double* rad = ctx.xfer + 1;
     double* nc = rad + ncell;
