@@ -86,7 +86,7 @@ struct Ctx {
   bool perm_valid = false;  // perm sorts the current slots by u cell
   bool perm_canonical = false;  // ... and within a cell by droplet (home)
   bool slots_sorted = false;    // the slots were last written in cell order
-  int since_reorder = 0;        // fused steps since then
+  int since_reorder = 0;        // steps since then, or since the droplets were put
   bool keys_valid = false;  // keys[cur] are the cells of the current positions
   double* col_tmp = nullptr;
   // bins
@@ -759,11 +759,25 @@ bool reorder_due() { return !ctx.slots_sorted || ctx.since_reorder + 1 >= kReord
 // the record columns are read and written at random through home.  1.5M
 // droplets on 96x80x64: an RK3 stage 401 -> 143 us, the coupling scatter
 // after it 453 -> 119 us, for a reordering of 490 us after a put (less later).
-// Populations below kSortSlotsMin stay as they are: their sort is bound by its
-// launches.  The amounts of a step are lost (slot order).
-constexpr int64_t kSortSlotsMin = 8192;
+// The amounts of a step are lost (slot order).
+//
+// Where the sort pays (us; slots as put and in cell order):
+// - From the second step after a put on, from 8192 droplets (three stages and
+//   the coupling 105 and 93 on 32^3, 128 and 114 on 96x80x64) and a 1024th of
+//   the cells (the sort scans them: 352 and 348 on 256x256x128).
+// - In the first pass only if it is paid back there, by the coupling update that
+//   follows where a coupling flag is set: from 32768 droplets (20k on 32^3 119 and 128
+//   for stages and coupling, 50k 143 and 144, 1M 1083 and 1217, but 3374 and 2547
+//   with interp before them and two more steps; 50k on 96x80x64 162 and 151) and a
+//   32nd of the cells (256x256x128: 100k 475 and 520, 300k 869 and 801).
+//   Without coupling the first three stages take 1793 and 2460 for 3M on 32^3.
+//   An interp that sorts takes longer itself (1M on 96x80x64 400 and 481) and what follows
+//   it less: with a fused step 952 and 673.
+constexpr int64_t kSortSlotsMin = 8192, kSortFirstMin = 32768;
 int sort_slots() {
-  if (!reorder_due() || ctx.n < kSortSlotsMin) return 0;
+  if (!reorder_due() || ctx.n < kSortSlotsMin || 1024 * ctx.n < ctx.ncell) return 0;
+  const bool first = !ctx.slots_sorted && ctx.since_reorder == 0;
+  if (first && (!src_mask() || ctx.n < kSortFirstMin || 32 * ctx.n < ctx.ncell)) return 0;
   CHK(flush_diag());
   if (!ctx.perm_valid || !ctx.keys_valid) CHK(bin_current(nullptr, nullptr, false));
   const int c = ctx.cur, d = 1 - c;
@@ -1285,6 +1299,7 @@ int ensure_capacity(int64_t n) {
   ctx.diag_mask = 0;
   ctx.amounts_valid = false;
   ctx.slots_sorted = false;
+  ctx.since_reorder = 0;
   ctx.perm_valid = false;
   ctx.keys_valid = false;
   return 0;
@@ -1670,8 +1685,10 @@ int ntlp_gpu_particle_update_rk3_prec(int32_t istage, int32_t it, int32_t prec) 
   CHK(check_prec(prec));
   if (istage < 1 || istage > 3) return fail(NTLP_E_INVALID, "istage must be 1, 2 or 3");
   if (ctx.n == 0) return NTLP_OK;
-  if (istage == 1 || !ctx.slots_sorted) CHK(sort_slots());
-  if (istage == 1) ctx.since_reorder++;
+  if (istage == 1) {
+    CHK(sort_slots());
+    ctx.since_reorder++;
+  }
   ctx.keys_valid = false;
   ctx.amounts_valid = false;
   StepArgs a = base_args();
