@@ -1600,18 +1600,19 @@ __global__ void __launch_bounds__(64 * kReduceWaves) k_xy_reduce(const double* p
 
 // Exclusive scan of the u-cell histogram: k_scan_reduce sums its tiles, then
 // k_scan_down<true> scans every tile locally and adds up the sums of the tiles
-// before it itself, which is cheaper than a launch (4.6 us) for a one-workgroup
-// scan of the sums up to kScanDirect tiles (1.3e8 cells; there the last
-// workgroups read 64 KB each); beyond, k_scan_bsum scans the sums and
-// k_scan_down<false> takes its tile's prefix from them.  With the counters
-// closed on the way, two launches a step fewer: 64^3 with 100k droplets (FP64)
-// 2100 -> 1982 us for 20 steps, 1000 droplets 684 -> 625 us for 10.  (Tile sums kept by the
-// step kernel, one atomic per wave and tile, made it 2 % slower at 20M droplets
-// and 9 % at 333k: every wave in flight adds to the same few words.)
+// before it itself; that work grows with the square of the tiles, so beyond
+// kScanDirect of them k_scan_bsum scans the sums in a launch between (one
+// workgroup) and k_scan_down<false> takes its tile's prefix from them.  Both
+// forms, us: 263 tiles (128^3) 13.3 and 14.4, 992 25.1 and 25.9, 2073 (256^3)
+// 48.8 and 47.6, 7872 184 and 178, 15453 (512x512x480) 358 and 344.  With the
+// counters closed on the way, two launches a step fewer: 64^3 with 100k droplets
+// (FP64) 2100 -> 1982 us for 20 steps, 1000 droplets 684 -> 625 us for 10.  (Tile
+// sums kept by the step kernel, one atomic per wave and tile, made it 2 % slower at
+// 20M droplets and 9 % at 333k: every wave in flight adds to the same few words.)
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
-constexpr int64_t kScanDirect = 16384;
+constexpr int64_t kScanDirect = 1400;
 
 __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave, int& total) {
   const int lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
