@@ -330,10 +330,13 @@ int to_host(void* dst, const void* src, size_t bytes) {
   return 0;
 }
 
-// The staging buffer with room for `room` doubles.  It is kept for the next
-// call, until the context is released or an allocation fails: allocated and
-// freed on each call it cost 40 to 260 us.  Its users leave it to the next in
-// stream order.
+// The staging buffer with room for `room` doubles.  Up to kXferKeep it is kept
+// for the next call, until the context is released or an allocation fails:
+// allocated and freed on each call it cost 40 to 260 us.  A larger one is given
+// back at the end of the call (Staged), for 1 % of its time (fields of 570 MB
+// each 62.4 ms kept, 63.4 given back).  Its users leave it to the next in stream
+// order.
+constexpr int64_t kXferKeep = 512ll << 20;
 int xfer_stage(int64_t room) {
   if (room <= ctx.xfer_cap) return 0;
   HIPCHK(hipStreamSynchronize(ctx.stream));
@@ -342,6 +345,12 @@ int xfer_stage(int64_t room) {
   ctx.xfer_cap = room;
   return 0;
 }
+
+struct Staged {
+  ~Staged() {
+    if (ctx.xfer_cap * (int64_t)sizeof(double) > kXferKeep) drop_staging();
+  }
+};
 
 // The device side of a droplet transfer: `want` doubles of the staging buffer;
 // where they are more than kXferBytes, or the device has no room for them, the
@@ -1247,6 +1256,7 @@ int ntlp_gpu_set_fields(const double* u, const double* v, const double* w, const
     if (!ctx.ext[f]) CHK(dalloc(ctx.ext[f], ctx.ext_elems, "ext field"));
   for (int f = 0; f < 3; ++f)
     if (!ctx.f32[f]) CHK(dalloc(ctx.f32[f], ctx.ext_elems, "fp32 field copy"));
+  Staged staged;
   if (layout != NTLP_LAYOUT_EXT) CHK(xfer_stage(in_elems));
   // one staging buffer serves the fields in turn, in stream order
   for (int f = 0; f < 5; ++f) {
@@ -1779,6 +1789,7 @@ int ntlp_gpu_apply_particle_coupling(double* T, double* q, int32_t layout) {
     return fail(NTLP_E_INVALID, "apply_particle_coupling takes x-pencil or core arrays");
   const int nx = ctx.g.nnx, ny = ctx.g.nny, nz = ctx.g.nnz;
   const int64_t elems = layout == NTLP_LAYOUT_XPENCIL ? (int64_t)(nx + 2) * ny * (nz + 2) : (int64_t)(nz + 2) * ny * nx;
+  Staged staged;
   int rc = xfer_stage(2 * elems);
   double* stage[2] = {ctx.xfer, ctx.xfer + elems};
   double* host[2] = {T, q};
@@ -1872,6 +1883,7 @@ int ntlp_gpu_wcell_counts(int32_t* num_array) {
   CHK(need_init());
   if (!num_array) return fail(NTLP_E_INVALID, "null output");
   const int64_t nw = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
+  Staged staged;
   CHK(xfer_stage((nw + 1) / 2));
   int32_t* d = reinterpret_cast<int32_t*>(ctx.xfer);
   if (ctx.n > 0 && wcell_runs()) {
@@ -1902,6 +1914,7 @@ int ntlp_gpu_calc_tauc_min(double* tauc_min) {
   const int64_t ncell = (int64_t)ctx.g.nnx * ctx.g.nny * ctx.g.nnz;
   const bool runs = wcell_runs();
   const int64_t room = runs ? 1 : 1 + 2 * ncell + (ncell + 1) / 2;
+  Staged staged;
   CHK(xfer_stage(room));
   unsigned long long* res = reinterpret_cast<unsigned long long*>(ctx.xfer);
   if (!runs) CHK(fill_f64(ctx.xfer, room, 0.0));
@@ -1935,6 +1948,7 @@ int ntlp_gpu_particle_xy_stats(double* s0, double* s1, double* lwp) {
   const int64_t nlw = (int64_t)ctx.g.nnx * ctx.g.nny, n0 = (int64_t)sh.rows * kStats0;
   const int64_t n1 = (int64_t)sh.rows * sh.nq_max * sh.nz2;
   const int64_t room = kStats0 + 24 * sh.nz2 + nlw + n0 + n1;
+  Staged staged;
   CHK(xfer_stage(room));
   double* out0 = ctx.xfer;
   double* out1 = out0 + kStats0;
