@@ -76,10 +76,6 @@ struct DevFields {
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-__device__ __forceinline__ int64_t ext_off(const DevFields& F, int k, int j, int i) {
-  return (int64_t)k + F.sj * (int64_t)(j + 1) + F.si * (int64_t)(i + 1);
-}
-
 // Number of leading elements of a(0:len-1) that are not greater than x, i.e.
 // the 0-based index of the first element > x, or len when there is none.  For
 // a monotone array this is exactly what Fortran's
@@ -606,16 +602,20 @@ __device__ __forceinline__ void lag_vertical(const double* lev, const int k[6], 
 // order of additions, FP64 in all precisions.  The out-of-domain branches with
 // first=last=0 leave the weights zero (the reference evaluates one stray
 // iteration outside its arrays there).
-// The weights stay in registers: every loop over them is unrolled, but for the
-// outermost over three pairs of levels, which shifts its lists down by two each
-// turn.  (Indexed by loop counters they lived in scratch memory, 1.2 KB a
-// droplet.)  The vector cache bounds it: a load of one level by a wave touches
-// about 21 cache lines, and the order of additions has the levels outermost, so
-// both levels of a pair come in one 16-byte load, and the upper one waits in a
-// register until the lower plane is summed.  FP64 step of 700k droplets on
-// 96^3 (280 us of it the tail of its few Levenberg-Marquardt solves): 1480 us
-// with scratch, about 900 with one level a load, 715 now; drawing them, in no
-// order: 11.9, 11.4 and 5.0 ms.
+// Every loop over the weights is unrolled, but for the outermost over three
+// pairs of levels, which shifts its lists down by two each turn, so that they can
+// stay in registers.  (Indexed by loop counters they lived in scratch memory, 1.2
+// KB a droplet.)  What the kernel around the gather keeps across it does not all
+// fit beside them: with 256 registers the BE steps spill 160 to 168 B a lane, the
+// RK3 steps 240 to 312, the single RK3 stages 208, the others 40 to 104.
+// The vector cache bounds it: a load of one level by a wave touches about 21
+// cache lines, and the order of additions has the levels outermost, so both
+// levels of a pair come in one 16-byte load, and the upper one waits in a
+// register until the lower plane is summed.  700k droplets on 96^3, FP64: a BE
+// step 1480 us with scratch, about 900 with one level a load, 715 now (280 of
+// each the tail of its few Levenberg-Marquardt solves; without such solves 1147
+// and 344), an RK3 step 2965 and 1025, mixed 2948 and 925; drawing them in put
+// order 11.9, 11.4 and 5.0 ms.
 __device__ __forceinline__ Fluid gather6_f64(const DevGrid& g, const DevFields& F, const double* s_z,
                                              const double* s_zz, double x, double y, double z,
                                              const Cell& c) {

@@ -50,8 +50,8 @@ __host__ __device__ __forceinline__ int64_t tix(int cols, int c, int64_t t) {
 __host__ __device__ __forceinline__ int64_t hix(int c, int64_t t) { return tix(kNHot, c, t); }
 // The six coupling amounts of a slot lie side by side: the scatters read them
 // through the cell sort, where a slot's neighbours are often another wave's, and
-// get them with two (FP32) or three 16-byte loads from a line or two instead of
-// six loads from six lines. The box scatter is bound by the latency of these
+// get their 24 (FP32) or 48 bytes with two or three loads from a line or two
+// instead of six loads from six lines. The box scatter is bound by the latency of these
 // loads and by its LDS adds: 395 -> 368 us for 6M droplets in FP64, 855 -> 846
 // for 20M with FP32 amounts; the steps that write them take the same time.
 __host__ __device__ __forceinline__ int64_t aix(int f, int64_t t) { return 6 * t + f; }
@@ -135,12 +135,6 @@ __device__ __forceinline__ int64_t xcd_block() {
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
 // --------------------------------------------------------------- tallies
-
-__device__ __forceinline__ long long wave_sum(long long v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // Newton tallies are summed per workgroup (ballots and 32-bit wave sums, then
 // LDS) and added to one of kTallySlots counter slots, each on its own cache

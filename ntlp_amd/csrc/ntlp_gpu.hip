@@ -1294,7 +1294,7 @@ int ensure_capacity(int64_t n) {
     CHK(dalloc(ctx.cold, kNCold * n, "cold state"));
     CHK(dalloc(ctx.pidx, n, "pidx"));
     CHK(dalloc(ctx.procidx, n, "procidx"));
-    CHK(dalloc(ctx.amounts, tiled_elems(n, 6), "coupling amounts"));
+    CHK(dalloc(ctx.amounts, 6 * n, "coupling amounts"));
     CHK(dalloc(ctx.diag, kNCold * n, "step diagnostics"));
     CHK(dalloc(ctx.keys[0], n, "keys"));
     CHK(dalloc(ctx.keys[1], n, "keys"));
