@@ -1989,7 +1989,8 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_serve_admit(AdmitAr
 // slots in order.  20M droplets on 256x256x128: 2.9 ms for the two kernels and
 // 1.28 ms for the first step.  Made in put order they took 9.3 ms, bound by the
 // cache lines of their random gathers (20 each), and the first step 8.6 ms to
-// read them through the sort.
+// read them through the sort.  Few droplets on a large grid, whose cells the sort
+// would all scan, are made in put order (perm and counts null).
 struct GenArgs {
   DevGrid g;
   DevConsts C;
@@ -2013,7 +2014,7 @@ struct GenArgs {
   int32_t* put_keys;    // u-cell keys in put order
   int32_t* keys;        // and in slot order
   int32_t* counts;
-  const int32_t* perm;  // slot -> droplet
+  const int32_t* perm;  // slot -> droplet (null: the same)
 };
 
 // the ensemble of droplet i: start[lo] <= i < start[lo + 1]
@@ -2056,7 +2057,7 @@ __global__ void __launch_bounds__(kBlock) k_gen_keys(GenArgs a) {
     a.procidx[i] = 0;
     for (int c = 0; c < kNCold; ++c) a.cold[(int64_t)c * a.cap + i] = 0.0;
   }
-  count_key(a.counts, key, valid);
+  if (a.counts) count_key(a.counts, key, valid);
 }
 
 template <int ILIN, bool ONE>
@@ -2066,7 +2067,7 @@ __global__ void __launch_bounds__(kBlock, kMinWaves<ILIN>) k_generate(GenArgs a)
   __syncthreads();
   const int64_t t = xcd_block() * kBlock + threadIdx.x;
   if (t >= a.n) return;
-  const int32_t i = a.perm[t];
+  const int32_t i = a.perm ? a.perm[t] : (int32_t)t;
   double kappa;
   int64_t mult;
   const NewDroplet nd = with_ensemble<ONE>(a, i, [&](const DevEnsemble& e, int64_t k) {

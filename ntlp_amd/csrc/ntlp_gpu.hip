@@ -1315,6 +1315,16 @@ int ensure_capacity(int64_t n) {
   return 0;
 }
 
+// Whether n droplets are drawn in cell order: not where the sort's scan of all
+// cells would take longer than the draw (50 us at 2^24 cells) for few droplets.
+// In put order and sorted, us: 1000 droplets on 512x512x480 45 and 420, with three
+// RK3 stages 140 and 535, with a fused step 2768 and 2776; 100k there 96 and 476,
+// 351 and 740, 3700 and 3662.  With more droplets the steps lose more than the draw
+// gains (300k on 400^3 224 and 453, with a step 2127 and 2043), on fewer cells there
+// is little to gain (1000 on 256x256x128 48 and 74).
+constexpr int64_t kGenScan = 1 << 24;
+bool gen_sorted(int64_t n) { return ctx.ncell <= kGenScan || 1024 * n >= ctx.ncell; }
+
 int check_ensemble(const ntlp_ensemble* e) {
   if (!e) return fail(NTLP_E_INVALID, "null ensemble");
   auto radius_ok = [](int kind, const double* p) {
@@ -1608,8 +1618,9 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
   a.procidx = ctx.procidx;
   a.put_keys = ctx.keys[1];
   a.keys = ctx.keys[0];
-  a.counts = ctx.counts;
-  a.perm = ctx.perm;
+  const bool sorted = gen_sorted(n);
+  a.counts = sorted ? ctx.counts : nullptr;
+  a.perm = sorted ? ctx.perm : nullptr;
   const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
   const bool lin = ctx.fl.ilin == 1;
   const bool one = nens == 1;
@@ -1617,7 +1628,7 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
     if (one) k_gen_keys<true><<<grid, kBlock, 0, ctx.stream>>>(a);
     else k_gen_keys<false><<<grid, kBlock, 0, ctx.stream>>>(a);
   });
-  if (!rc) rc = sort_keys(ctx.keys[1], nullptr);
+  if (!rc && sorted) rc = sort_keys(ctx.keys[1], nullptr);
   if (!rc)
     rc = launch("generate", [&] {
       if (lin && one) k_generate<1, true><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
@@ -1625,9 +1636,9 @@ int ntlp_gpu_particles_generate(const ntlp_ensemble* ens, const int64_t* counts,
       else if (one) k_generate<0, true><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
       else k_generate<0, false><<<grid8(n), kBlock, 0, ctx.stream>>>(a);
     });
-  if (!rc) {  // slots in cell order with their keys; uf, Tf and qinf wait in diag
-    ctx.home_identity = false;
-    ctx.slots_sorted = true;
+  if (!rc) {  // slots with their keys, in cell order if sorted; uf, Tf and qinf wait in diag
+    ctx.home_identity = !sorted;
+    ctx.slots_sorted = sorted;
     ctx.since_reorder = 0;
     ctx.keys_valid = true;
     ctx.diag_mask = kDiagFluid;
